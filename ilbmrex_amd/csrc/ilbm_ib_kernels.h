@@ -819,17 +819,20 @@ constexpr int kSumsBlock = 256;
 // Thread index and count of a block in linear order (x fastest), so that the
 // reductions below form the same wavefronts and trees in a block of
 // kSumsBlock x 1 threads and in one of the stream-collide kernel's 2D shapes.
+// Of a larger block the first kSumsBlock threads reduce.
 __device__ inline int lin_tid() { return (int)(threadIdx.x + threadIdx.y * blockDim.x); }
 __device__ inline int lin_nt() { return (int)(blockDim.x * blockDim.y); }
 
-__device__ __forceinline__ void sums_body(const IbArgs& a, int first_iter) {
+// F: the iteration's marker forces [3][nm]
+__device__ __forceinline__ void sums_body(const IbArgs& a, const double* F, int first_iter) {
   __shared__ double lds[6][16];
   const int nm = a.nm;
-  const int t = lin_tid(), nt = lin_nt();
+  const int t = lin_tid();
+  constexpr int nt = kSumsBlock;
   double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   const double z0 = (a.dim == 3) ? a.z0 : 0.0;
-  for (int m = t; m < nm; m += nt) {
-    const double fx = a.F[m] * a.dv, fy = a.F[nm + m] * a.dv, fz = a.F[2 * nm + m] * a.dv;
+  for (int m = t; m < nm && t < nt; m += nt) {
+    const double fx = F[m] * a.dv, fy = F[nm + m] * a.dv, fz = F[2 * nm + m] * a.dv;
     const double rx = a.xm[m] - a.x0, ry = a.xm[nm + m] - a.y0;
     const double rz = (a.dim == 3) ? a.xm[2 * nm + m] - z0 : 0.0;
     const double mx = ry * fz - rz * fy, my = rz * fx - rx * fz, mz = rx * fy - ry * fx;
@@ -839,18 +842,18 @@ __device__ __forceinline__ void sums_body(const IbArgs& a, int first_iter) {
   }
   for (int c = 0; c < 6; ++c) {
     const double r = wave_sum(acc[c]);
-    if ((t & 63) == 0) lds[c][t >> 6] = r;
+    if ((t & 63) == 0 && t < nt) lds[c][t >> 6] = r;
   }
   __syncthreads();
   if (t < 6) {
     double s = 0.0;
-    for (int wv = 0; wv < (nt + 63) / 64; ++wv) s += lds[t][wv];
+    for (int wv = 0; wv < nt / 64; ++wv) s += lds[t][wv];
     if (t < 3) a.sums[t] = first_iter ? s : a.sums[t] + s;
     else a.sums[t] = s;
   }
 }
 
-__global__ void __launch_bounds__(kSumsBlock) k_ib_sums(IbArgs a) { sums_body(a, a.first_iter); }
+__global__ void __launch_bounds__(kSumsBlock) k_ib_sums(IbArgs a) { sums_body(a, a.F, a.first_iter); }
 
 __device__ __forceinline__ void correct_body(const IbArgs& a, int64_t b) {
   if (b >= a.band_cells) return;
@@ -1432,21 +1435,22 @@ __global__ void __launch_bounds__(256) k_force_record(IbArgs a, RecArgs rec, int
 // record in one launch.
 __device__ __forceinline__ void sums_record_body(const IbArgs& a, const RecArgs& rec, int nblk) {
   __shared__ double lds[3][16];
-  sums_body(a, 1);
+  sums_body(a, a.F, 1);
   __syncthreads();
-  const int tid = lin_tid(), nt = lin_nt();
+  const int tid = lin_tid();
+  constexpr int nt = kSumsBlock;
   double acc[3] = {0.0, 0.0, 0.0};
-  for (int t = tid; t < nblk; t += nt)
+  for (int t = tid; t < nblk && tid < nt; t += nt)
     for (int c = 0; c < 3; ++c) acc[c] += rec.partial[(int64_t)c * nblk + t];
   for (int c = 0; c < 3; ++c) {
     const double r = wave_sum(acc[c]);
-    if ((tid & 63) == 0) lds[c][tid >> 6] = r;
+    if ((tid & 63) == 0 && tid < nt) lds[c][tid >> 6] = r;
   }
   __syncthreads();
   if (tid == 0) {
     double sum[3] = {0.0, 0.0, 0.0};
     for (int c = 0; c < 3; ++c)
-      for (int wv = 0; wv < (nt + 63) / 64; ++wv) sum[c] += lds[c][wv];
+      for (int wv = 0; wv < nt / 64; ++wv) sum[c] += lds[c][wv];
     write_force_record(a, rec, sum);
   }
 }
@@ -1498,6 +1502,517 @@ __global__ void __launch_bounds__(kBlock) k_step_record(StepArgs a, uint32_t tx,
   const int o2 = (a.sub_mode >= 2) ? a.sub_lo[2] : 0;
   step_body<LAT, ST, AM>(a, o0 + (int)(bx * blockDim.x + threadIdx.x),
                          wave_row(o1 + (int)(by * blockDim.y + threadIdx.y)), o2 + (int)bz, t, lds);
+}
+
+// ---------------------------------------------------------------------------
+// Body tiles: the direct forcing of a fixed 2D body inside the stream-collide
+// launch of the step before it.
+//
+// A step of a small level is bound by launches: interpolation, export and
+// stream-collide take 6.5, 8 and 10 us on the 512x256 FP64 cylinder, most of
+// it the launch and the first loads.  The cells under the marker stencils
+// (the level's non-empty band cells) are split into tiles of kBodyTile^2, one
+// block each at the front of the stream-collide launch of step s; the other
+// blocks leave those cells out (StepArgs::body_mask).  A tile updates its own
+// cells and computes, without storing them, the velocities of the further
+// cells its forcing depends on: the stencils of the markers that reach its
+// cells (and, over several iterations, of the markers that reach those).  So
+// after a barrier it has all it needs to interpolate, evaluate marker forces,
+// spread them to its cells and add the Guo term of step s + 1, with no
+// communication between blocks: a step is one launch.  Steps in us before and
+// after: cylinder 96x64 FP64 20.5 -> 11.4, 512x256 FP64 24.3 -> 13.8 and FP32
+// 18.0 -> 11.6, 391x203 FP32 with two iterations 49-52 -> 14.0, 512x256 IVC
+// 28.8 -> 19.4, the IVC cavity 39.4 -> 25.9.  (One block for the whole body
+// took 20 us for 650 cells, most of it serial rounds of loads.)  What is left
+// of a tile's chain on 512x256 FP64, in us: the pull and collision 5-6 (three
+// dependent loads and the FP64 divides), staging its lists 0.6,
+// interpolation 1.5, spreading 1.1, export 1.0, and 3 between two launches.
+// Every block reads only the previous buffer and the force of step s, and
+// writes the force of step s + 1 to the other of two slots, where the record
+// of step s + 1 finds it in the next launch.  The sums are those of
+// k_ib_interp, k_ib_ivc_*, k_ib_spread_t, k_ib_correct, k_ib_export_fixup and
+// k_sums_record term by term and in their order: the results are the same
+// bits.  An IVC body needs all markers between interpolation and spreading:
+// its tiles stop at the right-hand side and k_body_ivc does the rest.
+// ---------------------------------------------------------------------------
+constexpr int kBodyTile = 8;
+constexpr int kBodyOwn = kBodyTile * kBodyTile;   // a tile's own cells, at most (whole wavefronts)
+constexpr int kBodyLoops = 3;     // direct-forcing iterations, at most
+static_assert(kBodyOwn % 64 == 0 && kBodyOwn < kBlock, "own cells fill wavefronts and leave some");
+
+struct BodyTile {
+  int cell0, ncell[kBodyLoops];   // local cells: those of the stencils in iteration it (own cells first)
+  int nown;
+  int mk0, nmk[kBodyLoops];       // markers evaluated in iteration it
+  int gh0, ngh;                   // physical ghost cells of the stencils
+  int pt0;                        // [25][nmk[0]] local slots
+  int ep0;                        // entry offsets of the cells with entries (necell + 1)
+  int necell;
+  int ent0, nent;
+};
+
+struct BodyArgs {
+  IbArgs ib;              // F, Fband: the slot of the coming step
+  const BodyTile* tiles;
+  int ntile;
+  const int* cells;       // i | j << 16; the first kBlock of tile b at b * kBlock, the rest of the list at cell0
+  const int* mk;          // marker, kMkOwner set where this tile stores its U and F
+  const int* pt;
+  const int* eptr;
+  const int* em;          // local marker | group << 16
+  const double* ew;       // delta weight
+  const int* gh;          // local slot of the source | kind << 16 (0 copy, 1 value, 2 reflection)
+  const double* ghv;      // [2] boundary velocity
+  int lds;                // bytes of dynamic LDS
+};
+constexpr int kMkOwner = 1 << 30;
+
+// dynamic LDS of one tile: EulerVel slots, marker forces, target velocities
+// and weights, entries, lists
+__host__ __device__ inline int body_tile_lds(const BodyTile& T) {
+  const int nmk = T.nmk[0], nev = T.ncell[0] + T.ngh;
+  return 8 * (2 * nev + 16 * nmk + T.nent) + 4 * (T.nent + T.necell + 1 + 26 * nmk);
+}
+
+// MODE 0: stream-collide the tile's cells, then (forcing) the forcing of the
+// next step; an IVC body stops at the right-hand side.  MODE 1: the forcing
+// alone, on the macros of the band.  MODE 2: the IVC solve and the rest of
+// the forcing from the right-hand side.  gbuf: the buffer whose
+// post-collision populations get the Guo term (the step's output in MODE 0).
+template <class LAT, class ST, int AM, int MODE>
+__device__ __forceinline__ void body_tile(const StepArgs& s, const GridGeom& g, void* gbuf, double tau,
+                                          const BodyArgs& B, int tile, bool forcing, char* dyn) {
+  static_assert(LAT::D == 2, "2D bodies");
+  using T = typename ST::compute_t;
+  using R = typename ST::raw;
+  constexpr bool STEP = MODE == 0;
+  const IbArgs& a = B.ib;
+  const BodyTile& L = B.tiles[tile];
+  const int t = lin_tid(), lane = t & 63, wv = t >> 6;
+  const int nm = a.nm, nev = L.ncell[0] + L.ngh, nmk = L.nmk[0];
+  const int64_t bc = a.band_cells;
+  double* ev = reinterpret_cast<double*>(dyn);       // [2][nev]
+  double* Fl = ev + 2 * nev;                         // [3][nmk]
+  double* tl = Fl + 3 * nmk;                         // [3][nmk]
+  double* wl = tl + 3 * nmk;                         // [10][nmk]
+  double* ew = wl + 10 * nmk;                        // [nent]
+  int* em = reinterpret_cast<int*>(ew + L.nent);     // [nent]
+  int* ep = em + L.nent;                             // [necell + 1]
+  int* ml = ep + L.necell + 1;                       // [nmk]
+  int* pt = ml + nmk;                                // [25][nmk]
+  // this thread's cell: the own cells on the first wavefront, further
+  // stencil cells on the others
+  const int ij0 = B.cells[tile * kBlock + t];
+  // the tile's lists, loaded beside the cell's populations
+  constexpr int kPre = 3;
+  double pw[kPre] = {}, pe[kPre] = {};
+  int pm[kPre] = {}, pp[kPre] = {}, pep = 0;
+  double ptv[3] = {};
+  int pmk = 0;
+  const bool lists = !STEP || forcing;
+  if (lists) {
+    if (t < nmk) pmk = B.mk[L.mk0 + t];
+#pragma unroll
+    for (int r = 0; r < kPre; ++r) {
+      const int x = t + r * kBlock;
+      if (x < L.nent) { pe[r] = B.ew[L.ent0 + x]; pm[r] = B.em[L.ent0 + x]; }
+      if (MODE != 2 && x < 25 * nmk) pp[r] = B.pt[L.pt0 + x];
+    }
+    if (t <= L.necell) pep = B.eptr[L.ep0 + t];
+    if (MODE != 2) {
+#pragma unroll
+      for (int r = 0; r < kPre; ++r) {
+        const int x = t + r * kBlock;
+        if (x < 10 * nmk) {
+          const int q = x / nmk;
+          pw[r] = a.wts[q * nm + (B.mk[L.mk0 + x - q * nmk] & ~kMkOwner)];
+        }
+      }
+      if (t < nmk) target_velocity(a, pmk & ~kMkOwner, &ptv[0], &ptv[1], &ptv[2]);
+    }
+  }
+  CellOut<LAT, ST> own;
+  const int own_i = ij0 & 0xffff, own_j = ij0 >> 16;
+  auto band_of = [&](int i, int j) { return (int64_t)(j - a.band_lo[1]) * a.band_n[0] + (i - a.band_lo[0]); };
+  const int64_t own_b = band_of(own_i, own_j);
+  if (t < L.nown) {
+    if constexpr (STEP) {
+      T f[LAT::Q];
+      StepOff<AM> self;
+      step_load<LAT, ST, AM>(s, own_i, own_j, 0, f, self);
+      (void)step_update<LAT, ST, AM>(s, own_i, own_j, 0, f, self, &own);
+    } else {
+      for (int c = 0; c < 4; ++c) own.mac[c] = a.Mband[c * bc + own_b];
+      const int64_t self = g.idx(own_i, own_j, a.band_lo[2]);
+#pragma unroll
+      for (int q = 0; q < LAT::Q; ++q)
+        own.post[q] = ST::load(static_cast<const R*>(gbuf), (int64_t)q * g.qs + self, T(LAT::w[q]));
+    }
+    if (MODE != 2) {
+      ev[t] = own.mac[1];
+      ev[nev + t] = own.mac[2];
+    }
+  }
+  if (MODE != 2 && lists && t >= kBodyOwn) {
+    constexpr int kSt = kBlock - kBodyOwn;
+    for (int ci = L.nown + t - kBodyOwn; ci < L.ncell[0]; ci += kSt) {
+      const int ij = (ci < L.nown + kSt) ? ij0 : B.cells[L.cell0 + ci - (L.nown + kSt)];
+      const int i = ij & 0xffff, j = ij >> 16;
+      double u, v;
+      if constexpr (STEP) {
+        T f[LAT::Q];
+        StepOff<AM> self;
+        CellOut<LAT, ST> o;
+        step_load<LAT, ST, AM>(s, i, j, 0, f, self);
+        (void)step_update<LAT, ST, AM, false>(s, i, j, 0, f, self, &o);
+        u = o.mac[1];
+        v = o.mac[2];
+      } else {
+        u = a.Mband[bc + band_of(i, j)];
+        v = a.Mband[2 * bc + band_of(i, j)];
+      }
+      ev[ci] = u;
+      ev[nev + ci] = v;
+    }
+  }
+  if (lists) {
+#pragma unroll
+    for (int r = 0; r < kPre; ++r) {
+      const int x = t + r * kBlock;
+      if (x < L.nent) { ew[x] = pe[r]; em[x] = pm[r]; }
+      if (MODE != 2 && x < 25 * nmk) pt[x] = pp[r];
+      if (MODE != 2 && x < 10 * nmk) wl[x] = pw[r];
+    }
+    if (t <= L.necell) ep[t] = pep;
+    if (t < nmk) {
+      ml[t] = pmk;
+      for (int c = 0; c < 3; ++c) tl[c * nmk + t] = ptv[c];
+    }
+    for (int x = t + kPre * kBlock; x < L.nent; x += kBlock) { ew[x] = B.ew[L.ent0 + x]; em[x] = B.em[L.ent0 + x]; }
+    for (int x = t + kBlock; x <= L.necell; x += kBlock) ep[x] = B.eptr[L.ep0 + x];
+    for (int x = t + kBlock; x < nmk; x += kBlock) {
+      ml[x] = B.mk[L.mk0 + x];
+      double tv[3];
+      target_velocity(a, ml[x] & ~kMkOwner, &tv[0], &tv[1], &tv[2]);
+      for (int c = 0; c < 3; ++c) tl[c * nmk + x] = tv[c];
+    }
+    if (MODE != 2) {
+      for (int x = t + kPre * kBlock; x < 25 * nmk; x += kBlock) pt[x] = B.pt[L.pt0 + x];
+      for (int x = t + kPre * kBlock; x < 10 * nmk; x += kBlock) {
+        const int q = x / nmk;
+        wl[x] = a.wts[q * nm + (B.mk[L.mk0 + x - q * nmk] & ~kMkOwner)];
+      }
+    }
+  }
+  if (!lists) return;
+  __syncthreads();
+  if (MODE != 2 && L.ngh) {
+    // FillPatch velocities of the ghost cells (macro_fill)
+    for (int x = t; x < 2 * L.ngh; x += kBlock) {
+      const int c = x >= L.ngh ? 1 : 0, gi = x - c * L.ngh;
+      const int code = B.gh[L.gh0 + gi], kind = code >> 16;
+      const double m = ev[c * nev + (code & 0xffff)], bv = B.ghv[2 * (L.gh0 + gi) + c];
+      ev[c * nev + L.ncell[0] + gi] = (kind == 0) ? m : (kind == 1) ? bv : 2.0 * bv - m;
+    }
+    __syncthreads();
+  }
+  const double d = a.dx[0] * a.dx[1];
+  double eft[2] = {0.0, 0.0};
+  for (int it = 0; it < a.nloop; ++it) {
+    const int nmi = L.nmk[it];
+    double* Fg = a.F + (int64_t)(a.nloop - 1 - it) * 3 * nm;   // the last iteration's first
+    // component c of local marker x: its velocity to U, force (or IVC
+    // right-hand side); c = 0 also takes the z component, whose velocity is 0
+    auto marker_force = [&](int x, int c, double vel) {
+      const int mo = ml[x], m = mo & ~kMkOwner;
+      const bool keep = (mo & kMkOwner) != 0;
+      double denom = a.dt;
+      if (a.coupling == 2) {
+        // explicit_force_tv's diagonal
+        const double dV = a.dx[0] * a.dx[1];
+        double s2 = 0.0;
+#pragma unroll 1
+        for (int p = 0; p < 25; ++p) {
+          const int ip = a.base[m] + p / 5 - 2, jp = a.base[nm + m] + p % 5 - 2;
+          if (ip < a.dlo[0] || ip > a.dhi[0] || jp < a.dlo[1] || jp > a.dhi[1]) continue;
+          const double dval = wl[(p / 5) * nmk + x] * wl[(5 + p % 5) * nmk + x];
+          s2 += dval * dval * dV;
+        }
+        denom = a.dt * fmax(a.dv * s2, a.diag_eps);
+      }
+      auto put = [&](int k, double target, double v) {
+        if (keep) a.U[k * nm + m] = v;
+        if (a.use_ivc) {
+          if (keep) a.rhs[k * nm + m] = (target - v) / a.dt;
+          return;
+        }
+        double F = 0.0;
+        F += a.relax * (target - v) / denom;
+        Fl[k * nmk + x] = F;
+        if (keep) Fg[k * nm + m] = F;
+      };
+      put(c, tl[c * nmk + x], vel);
+      if (c == 0) put(2, tl[2 * nmk + x], 0.0);
+    };
+    if constexpr (MODE == 2) {
+      // k_ib_ivc_matvec's rows of the tile's markers, kRow of a wavefront at a time
+      constexpr int kRow = 4, nw = kBlock / 64;
+      for (int x0 = wv; x0 < nmi; x0 += kRow * nw) {
+        double sx[kRow] = {}, sy[kRow] = {}, sz[kRow] = {};
+        int row[kRow];
+#pragma unroll
+        for (int k = 0; k < kRow; ++k) row[k] = ml[x0 + k * nw < nmi ? x0 + k * nw : x0];
+        for (int jj = lane; jj < nm; jj += 64) {
+          const double r0 = a.rhs[jj], r1 = a.rhs[nm + jj], r2 = a.rhs[2 * nm + jj];
+#pragma unroll
+          for (int k = 0; k < kRow; ++k) {
+            const double aij = a.Ainv[(int64_t)(row[k] & ~kMkOwner) * nm + jj];
+            sx[k] += aij * r0;
+            sy[k] += aij * r1;
+            sz[k] += aij * r2;
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < kRow; ++k) {
+          sx[k] = wave_sum(sx[k]); sy[k] = wave_sum(sy[k]); sz[k] = wave_sum(sz[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kRow; ++k) {
+          const int x = x0 + k * nw;
+          if (lane != 0 || x >= nmi) continue;
+          const double F0 = 0.0 + sx[k], F1 = 0.0 + sy[k], F2 = 0.0 + sz[k];
+          Fl[x] = F0; Fl[nmk + x] = F1; Fl[2 * nmk + x] = F2;
+          if (row[k] & kMkOwner) {
+            const int m = row[k] & ~kMkOwner;
+            a.F[m] = F0; a.F[nm + m] = F1; a.F[2 * nm + m] = F2;
+          }
+        }
+      }
+    } else if (a.tree) {
+      // 16 lanes per marker, as interp_group_body<2>
+      const int sub = t & 15;
+      for (int x0 = 0; x0 < nmi; x0 += kBlock / 16) {   // uniform rounds: every lane shuffles
+        const int x = x0 + (t >> 4), xc = x < nmi ? x : 0;
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+          const int p = sub + 16 * r, pc = p < 25 ? p : 0;
+          const int slot = pt[pc * nmk + xc];
+          const double dv = wl[(pc / 5) * nmk + xc] * wl[(5 + pc % 5) * nmk + xc];
+          const double e0 = ev[slot], e1 = ev[nev + slot];
+          if (p < 25) {
+            s0 += dv * d;
+            s1 += dv * e0 * d;
+            s2 += dv * e1 * d;
+          }
+        }
+        s0 = row_sum16(s0);
+        s1 = row_sum16(s1);
+        s2 = row_sum16(s2);
+        if (x < nmi && sub < 2) {
+          double u = sub ? s2 : s1;
+          if (a.renorm_interp && s0 > 0.0) u /= s0;
+          marker_force(x, sub, u);
+        }
+      }
+    } else {
+      // serial order over the stencil, as interp_body; a lane per component
+      for (int y = t; y < 2 * nmi; y += kBlock) {
+        const int c = y >= nmi ? 1 : 0, x = y - c * nmi;
+        double part = 0.0, u = 0.0;
+#pragma unroll 1
+        for (int ii = 0; ii < 5; ++ii) {   // a stencil row's reads are in flight together
+          double e[5], tv[5];
+#pragma unroll
+          for (int jj = 0; jj < 5; ++jj) {
+            e[jj] = ev[c * nev + pt[(5 * ii + jj) * nmk + x]];
+            tv[jj] = wl[(5 + jj) * nmk + x];
+          }
+          const double tu = wl[ii * nmk + x];
+#pragma unroll
+          for (int jj = 0; jj < 5; ++jj) {
+            const double dv = tu * tv[jj];
+            part += dv * d;
+            u += dv * e[jj] * d;
+          }
+        }
+        if (a.renorm_interp && part > 0.0) u /= part;
+        double U0 = 0.0;
+        U0 += u;
+        marker_force(x, c, U0);
+      }
+    }
+    if (MODE != 2 && a.use_ivc) return;
+    __syncthreads();
+    // spreading to the cells the next iteration reads, or to the own cells
+    // (spread_cell_sum)
+    const bool last = it == a.nloop - 1;
+    const int nupd = last ? L.nown : L.ncell[it + 1];
+    for (int ci = t; ci < nupd; ci += kBlock) {
+      constexpr int kB = 4;   // entries whose reads are in flight together
+      const int e0 = ep[ci], e1 = ep[ci + 1];
+      double tot[2] = {0.0, 0.0}, gs[2] = {0.0, 0.0};
+      int cur = 0;
+      for (int e = e0; e < e1; e += kB) {
+        int mg[kB];
+        double dd[kB], f0[kB], f1[kB];
+#pragma unroll
+        for (int q = 0; q < kB; ++q) {
+          const int ee = (e + q < e1) ? e + q : e0;
+          mg[q] = em[ee];
+          dd[q] = ew[ee];
+        }
+#pragma unroll
+        for (int q = 0; q < kB; ++q) {
+          f0[q] = Fl[mg[q] & 0xffff];
+          f1[q] = Fl[nmk + (mg[q] & 0xffff)];
+        }
+#pragma unroll
+        for (int q = 0; q < kB; ++q) {
+          if (e + q >= e1) break;
+          const int grp = mg[q] >> 16;
+          const double p0 = dd[q] * (f0[q] * a.dv), p1 = dd[q] * (f1[q] * a.dv);
+          if (grp != cur) {
+            if (cur != 0) { tot[0] += gs[0]; tot[1] += gs[1]; }
+            gs[0] = gs[1] = 0.0;
+            cur = grp;
+          }
+          if (cur == 0) { tot[0] += p0; tot[1] += p1; }
+          else { gs[0] += p0; gs[1] += p1; }
+        }
+      }
+      if (cur != 0) { tot[0] += gs[0]; tot[1] += gs[1]; }
+      if (ci < L.nown) {   // ci == t
+        eft[0] += tot[0];
+        eft[1] += tot[1];
+      }
+      if (!last) {
+        ev[ci] += a.dt * tot[0];
+        ev[nev + ci] += a.dt * tot[1];
+      }
+    }
+    if (!last) __syncthreads();
+  }
+  if (t < L.nown) {
+    // k_ib_export_fixup
+    const double rho = own.mac[0];
+    const double fx = a.dt * rho * eft[0], fy = a.dt * rho * eft[1], fz = a.dt * rho * 0.0;
+    a.Fband[own_b] = fx;
+    a.Fband[bc + own_b] = fy;
+    a.Fband[2 * bc + own_b] = fz;
+    if (!(fx == 0.0 && fy == 0.0 && fz == 0.0)) {
+      R* gb = static_cast<R*>(gbuf);
+      const int64_t self = g.idx(own_i, own_j, a.band_lo[2]);
+      const T ux = T(own.mac[1]), uy = T(own.mac[2]), uz = T(own.mac[3]);
+      const T fac = T(1.0) - T(0.5) / T(tau);
+#pragma unroll
+      for (int q = 0; q < LAT::Q; ++q) {
+        T gq = own.post[q];
+        gq += guo_q<LAT, T>(q, fac, ux, uy, uz, T(fx), T(fy), T(fz));
+        ST::store(gb, (int64_t)q * g.qs + self, gq, T(LAT::w[q]));
+      }
+    }
+  }
+}
+
+// The record of a body-tile step, one block: the marker sums of every
+// iteration, then the export's block sums from the force of the step (64
+// band cells per wavefront, four wavefronts in order, as the 256-thread
+// export blocks add them) and their sum as sums_record_body adds it.
+// dyn: 8 * 8 * nblk bytes.
+__device__ __forceinline__ void body_record(const IbArgs& a, const RecArgs& rec, char* dyn) {
+  __shared__ double lds[3][4];
+  const int t = lin_tid(), lane = t & 63, wv = t >> 6;
+  const int64_t bc = a.band_cells;
+  const int nblk = (int)((bc + 255) / 256);
+  double* wsum = reinterpret_cast<double*>(dyn);   // [2][4][nblk]
+  constexpr int kC = 8;   // blocks whose loads are in flight together
+  for (int b0 = 0; b0 < nblk; b0 += kC) {
+    double v[kC][2];
+#pragma unroll
+    for (int k = 0; k < kC; ++k) {
+      const int64_t b = (int64_t)(b0 + k) * 256 + t;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) v[k][c] = (b < bc) ? a.Fband[c * bc + b] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < kC; ++k)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const double r = wave_sum(v[k][c]);
+        if (lane == 0 && b0 + k < nblk) wsum[(c * 4 + wv) * nblk + b0 + k] = r;
+      }
+  }
+  for (int it = 0; it < a.nloop; ++it) {
+    sums_body(a, a.F + (int64_t)(a.nloop - 1 - it) * 3 * a.nm, it == 0);
+    __syncthreads();
+  }
+  double acc[2] = {0.0, 0.0};
+  for (int b = t; b < nblk; b += kSumsBlock)
+    for (int c = 0; c < 2; ++c) {
+      double s = 0.0;
+      for (int w = 0; w < 4; ++w) s += wsum[(c * 4 + w) * nblk + b];
+      acc[c] += s;
+    }
+  for (int c = 0; c < 2; ++c) {
+    const double r = wave_sum(acc[c]);
+    if (lane == 0) lds[c][wv] = r;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double sum[3] = {0.0, 0.0, 0.0};
+    for (int c = 0; c < 2; ++c)
+      for (int w = 0; w < 4; ++w) sum[c] += lds[c][w];
+    write_force_record(a, rec, sum);
+  }
+}
+
+__global__ void k_gather_doubles(const double* src, const int* idx, double* dst, int64_t n) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) dst[t] = src[idx[t]];
+}
+
+// The forcing alone, a block per tile (MODE 1: the first step of an advance,
+// with blocks of 256 band cells behind that write the exported force of the
+// cells outside the tiles; MODE 2: the IVC solve and spreading of any step).
+template <class LAT, class ST, int MODE>
+__global__ void __launch_bounds__(kBlock) k_body(BodyArgs B, const unsigned char* mask, GridGeom g, void* gbuf,
+                                                 double tau) {
+  extern __shared__ char dyn[];
+  if (MODE == 1 && blockIdx.x >= (unsigned)B.ntile) {
+    const int64_t b = (int64_t)(blockIdx.x - B.ntile) * kBlock + threadIdx.x;
+    if (b < B.ib.band_cells && !mask[b])
+      for (int c = 0; c < 3; ++c) B.ib.Fband[c * B.ib.band_cells + b] = B.ib.dt * B.ib.Mband[b] * 0.0;
+    return;
+  }
+  body_tile<LAT, ST, kAddrWall64, MODE>(StepArgs{}, g, gbuf, tau, B, blockIdx.x, true, dyn);
+}
+
+// A step's stream-collide with the forcing of the step after it in its first
+// blocks (which with forcing == 0 only update their cells), then the force
+// record of its own forcing (ia, rec); the other blocks are k_step's in
+// linear order, tw cells wide (k_step's block width; of the 256 threads a
+// width of 192 leaves the last wavefront idle).  The chains of dependent loads and reductions come first and
+// run beside the others.
+static_assert(kBlock == kSumsBlock, "the record block of a step launch");
+template <class LAT, class ST, int AM>
+__global__ void __launch_bounds__(kBlock) k_step_body(StepArgs a, uint32_t tx, uint32_t tw, IbArgs ia, RecArgs rec,
+                                                      BodyArgs B, int forcing) {
+  extern __shared__ char dyn[];
+  __shared__ double lds[kBlock / 64];
+  const uint32_t nb = (uint32_t)B.ntile;
+  if (blockIdx.x < nb) {
+    body_tile<LAT, ST, AM, 0>(a, a.g, a.gout, a.tau, B, blockIdx.x, forcing != 0, dyn);
+    return;
+  }
+  if (blockIdx.x == nb) {
+    body_record(ia, rec, dyn);
+    return;
+  }
+  const uint32_t t = blockIdx.x - nb - 1;
+  const uint32_t by = t / tx, bx = t - by * tx;
+  step_body_masked<LAT, ST, AM>(a, threadIdx.x < tw, (int)(bx * tw + threadIdx.x),
+                                wave_row((int)(by * blockDim.y + threadIdx.y)), t, lds);
 }
 
 // The ComputeIBForce record (AmrCoreLBM.cpp:456-631) from the band sum of
@@ -1613,7 +2128,7 @@ __global__ void __launch_bounds__(kSumsBlock) k_ib_sums_b(const IbCase* __restri
                                                     int it) {
   const IbArgs& a = A[map[blockIdx.x].c].ib;
   if (it >= a.nloop || a.nloop == 1) return;
-  sums_body(a, it == 0);
+  sums_body(a, a.F, it == 0);
 }
 
 __global__ void k_ib_correct_b(const IbCase* __restrict__ A, const BlockRef* __restrict__ map, int it) {

@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <new>
 #include <string>
@@ -308,6 +309,10 @@ using FixFn = void (*)(int, dim3, dim3, hipStream_t, const IbArgs&, const GridGe
 using GhostFn = void (*)(dim3, dim3, hipStream_t, const GhostArgs&);
 using GhostRecFn = void (*)(unsigned, hipStream_t, const GhostArgs&, unsigned, const IbArgs&, const RecArgs&, int);
 using StepRecFn = void (*)(dim3, dim3, hipStream_t, const StepArgs&, const IbArgs&, const RecArgs&, int);
+// body tiles (2D): a step with the next forcing, and the forcing alone
+using StepBodyFn = void (*)(dim3, dim3, hipStream_t, const StepArgs&, const IbArgs&, const RecArgs&, const BodyArgs&,
+                            bool);
+using BodyFn = void (*)(int, hipStream_t, const BodyArgs&, const unsigned char*, const GridGeom&, void*, double);
 
 // the stream-collide kernels take a wavefront's row as uniform (wave_row)
 static void check_step_block(dim3 b) {
@@ -363,6 +368,38 @@ static void launch_step_rec(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, co
   check_step_block(b);
   const uint32_t nt = g.x * g.y * g.z;
   hipLaunchKernelGGL((k_step_record<LAT, ST, AM>), dim3(nt + 1), b, 0, s, a, g.x, g.y, nt, ia, r, nblk);
+}
+
+// g, b: k_step's grid and block
+template <class LAT, class ST, int AM>
+static void launch_step_body(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, const IbArgs& ia, const RecArgs& r,
+                             const BodyArgs& B, bool forcing) {
+  check_step_block(b);
+  if (g.z != 1 || (b.x * b.y != (unsigned)kBlock && b.y != 1))
+    throw StatusError{ILBM_ERR_INVALID, "body step block must hold 256 threads or one row"};
+  hipLaunchKernelGGL((k_step_body<LAT, ST, AM>), dim3(g.x * g.y + 1 + (unsigned)B.ntile), dim3(kBlock / b.y, b.y),
+                     (size_t)B.lds, s, a, g.x, b.x, ia, r, B, forcing ? 1 : 0);
+}
+// mode 1: the forcing (of an IVC body its first half), 2: an IVC body's second half
+template <class LAT, class ST>
+static void launch_body(int mode, hipStream_t s, const BodyArgs& B, const unsigned char* mask, const GridGeom& g,
+                        void* gbuf, double tau) {
+  const unsigned nt = (unsigned)B.ntile, nb = (unsigned)((B.ib.band_cells + kBlock - 1) / kBlock);
+  const dim3 blk(kBlock);
+  if (mode == 2) hipLaunchKernelGGL((k_body<LAT, ST, 2>), dim3(nt), blk, (size_t)B.lds, s, B, mask, g, gbuf, tau);
+  else hipLaunchKernelGGL((k_body<LAT, ST, 1>), dim3(nt + nb), blk, (size_t)B.lds, s, B, mask, g, gbuf, tau);
+}
+
+// the body-tile launches of a 2D class (none in 3D)
+template <class ST>
+static void pick_body(int lat, int am, StepBodyFn& sbf, BodyFn& bf) {
+  sbf = nullptr;
+  bf = nullptr;
+  if (lat != 0) return;
+  sbf = (am == kAddrWrap) ? launch_step_body<D2Q9, ST, kAddrWrap>
+      : (am == kAddrWallX32) ? launch_step_body<D2Q9, ST, kAddrWallX32>
+      : (am == kAddrWall32) ? launch_step_body<D2Q9, ST, kAddrWall32> : launch_step_body<D2Q9, ST, kAddrWall64>;
+  bf = launch_body<D2Q9, ST>;
 }
 
 template <class LAT, class ST>
@@ -452,6 +489,19 @@ constexpr int kFarBlocksPerCu = 0;
 constexpr int kFarAfter = 0;
 constexpr int kRingStream = 0;   // Level::RING_NEAR
 
+// Dynamic LDS a body tile may take: the stream-collide blocks of the launch
+// get it too (8 blocks of 256 threads fill a CU).
+constexpr int kBodyLds = 20 * 1024;
+// Levels of reduced storage take body tiles up to this many cells, FP64
+// levels at every size.  The tiles' registers leave the stream-collide
+// blocks of their launch 4 waves per SIMD instead of 7-8, which large
+// levels of small populations feel, and the overlapped step is there for
+// them.  Steps in us, body tiles / the path without them: FP64 512x256
+// 13.8 / 24.3, 2000x1000 57 / 78, 3000x3000 237 / 256; FP32 512x256 11.6 /
+// 18.0, 1000x1000 22 / 31, 2000x1000 37 / 44, 2400x1250 54 / 52, 2000x2000
+// 69 / 67; FP16-shifted 2000x1000 32 / 43, 2400x2000 72 / 56.
+constexpr int64_t kBodyReducedCells = (int64_t)5 << 19;
+
 struct Level {
   ilbm_case_desc c{};
   int lat = -1, st = -1;
@@ -473,6 +523,17 @@ struct Level {
   GhostFn ghostfn = nullptr;
   GhostRecFn ghostrecfn = nullptr;
   StepRecFn steprecfn = nullptr;
+  StepBodyFn stepbodyfn = nullptr;
+  BodyFn bodyfn = nullptr;
+  // body tiles (see body_tile): their tables, the mask of their cells in the
+  // band, and the second slot of force and export
+  bool body_ok = false;
+  unsigned char* body_mask = nullptr;
+  int* body_int = nullptr;
+  double* body_dbl = nullptr;
+  BodyTile* body_tiles = nullptr;
+  BodyArgs body{};              // the tables' part
+  double *body_F = nullptr, *body_Fband = nullptr;
   // the step's marker kinematics were launched with another kernel (an AMR
   // level's coarse-fine ghost fill); the next forcing skips its own launch
   bool moved_ext = false;
@@ -548,6 +609,7 @@ struct Level {
   int64_t nent = 0, ent_cap = 0;
   double* frstate_d = nullptr;
   std::vector<double> xm_h, ut_h;
+  std::vector<int> ne_h, nee_h, em_h, ec_h;   // the spreading lists on the host
   bool moving = false;
   bool dev_kin = false;          // moving body advanced on the device (explicit forcing)
   double* xref_d = nullptr;      // [2][nm] section outline in body coordinates
@@ -650,6 +712,7 @@ struct Level {
     dev_free(xm_d); dev_free(ut_d); dev_free(U_d); dev_free(F_d); dev_free(Mm_d);
     dev_free(base_d); dev_free(wts_d); dev_free(scale_d); dev_free(rhs_d); dev_free(sums_d);
     dev_free(Ainv_d); dev_free(rowptr_d); dev_free(entm_d); dev_free(entc_d); dev_free(entw_d); dev_free(frstate_d);
+    dev_free(body_mask); dev_free(body_int); dev_free(body_dbl); dev_free(body_tiles); dev_free(body_F); dev_free(body_Fband);
     dev_free(ne_d); dev_free(nee_d); dev_free(fpartial); dev_free(clock_d); dev_free(xref_d); dev_free(chunk_d);
     for (int b = 0; b < 2; ++b) { dev_free(Mw[b]); dev_free(Dw[b]); }
     if (stream && own_stream) (void)hipStreamDestroy(stream);
@@ -794,6 +857,9 @@ struct Level {
     if (lat == 0) pk(D2Q9{});
     else if (lat == 1) pk(D3Q19{});
     else pk(D3Q27{});
+    if (st == 0) pick_body<StF64>(lat, am, stepbodyfn, bodyfn);
+    else if (st == 1) pick_body<StF32>(lat, am, stepbodyfn, bodyfn);
+    else pick_body<StF16S>(lat, am, stepbodyfn, bodyfn);
     tau = 3.0 * c.nu / c.dx[0] + 0.5;  // AmrCoreLBM.cpp:225
     dt = c.dx[0];                       // AmrCoreLBM.cpp:228
   }
@@ -885,7 +951,7 @@ struct Level {
     xm_d = dev_alloc<double>(3 * nm);
     ut_d = dev_alloc<double>(3 * nm);
     U_d = dev_alloc<double>(3 * nm);
-    F_d = dev_alloc<double>(3 * nm);
+    F_d = dev_alloc<double>(3 * (size_t)nm * std::max(c.loop_ns, 1));   // body tiles keep every iteration's
     Mm_d = dev_alloc<double>(3 * nm);
     base_d = dev_alloc<int>(3 * nm);
     wts_d = dev_alloc<double>(15 * nm);
@@ -904,7 +970,251 @@ struct Level {
     fpartial_n = 3 * ((band_cells + 255) / 256 + band_cells / kSpreadWaves + tiles + 2);
     fpartial = dev_alloc<double>(fpartial_n);
     upload_markers();
+    setup_body();
     ncol = (c.dim == 3) ? 33 : 23;
+  }
+
+  // The source of a stencil point outside the walls as macro_fill resolves
+  // it: kind 0 a copy of `cell`, 1 the value v, 2 the reflection 2 v - cell.
+  struct GhostSrc {
+    int kind;
+    int cell[2];
+    double v[2];
+  };
+  GhostSrc ghost_src(const int iv[2]) const {
+    GhostSrc r{1, {0, 0}, {0.0, 0.0}};
+    int p[2] = {iv[0], iv[1]};
+    for (int iter = 0; iter < 8; ++iter) {
+      int side[2] = {0, 0};   // 1 low, 2 high
+      bool any = false, wall = false;
+      for (int d = 0; d < 2; ++d) {
+        side[d] = (p[d] < 0) ? 1 : (p[d] > c.n[d] - 1) ? 2 : 0;
+        if (side[d]) { any = true; wall = wall || !c.periodic[d]; }
+      }
+      if (!any) { r.kind = 0; r.cell[0] = p[0]; r.cell[1] = p[1]; return r; }
+      if (!wall) {
+        for (int d = 0; d < 2; ++d) p[d] += (side[d] == 1) ? c.n[d] : (side[d] == 2) ? -c.n[d] : 0;
+        continue;
+      }
+      auto type = [&](int d) { return side[d] == 1 ? c.bc_lo[d] : side[d] == 2 ? c.bc_hi[d] : -1; };
+      for (int want : {(int)BC_USER_2, (int)BC_USER_1, (int)BC_EXT_DIR})
+        for (int d = 0; d < 2; ++d) {
+          if (type(d) != want) continue;
+          const double* bv = (side[d] == 1) ? c.bc_lo_val[d] : c.bc_hi_val[d];
+          r.v[0] = bv[1];
+          r.v[1] = bv[2];
+          r.kind = (want == BC_USER_2) ? 2 : 1;
+          for (int e = 0; e < 2; ++e) r.cell[e] = std::min(std::max(p[e], 0), c.n[e] - 1);
+          return r;
+        }
+      int sel = -1;
+      for (int d = 0; d < 2; ++d)
+        if (type(d) == BC_FOEXTRAP) sel = d;
+      if (sel < 0) return r;
+      p[sel] = (side[sel] == 1) ? 0 : c.n[sel] - 1;
+    }
+    return r;
+  }
+
+  // Tables of the body tiles of a fixed 2D body (ILBM_BODY_TILES=0 keeps the
+  // separate forcing kernels).  A body they cannot hold -- stencils beyond
+  // the ghost layers, lists over the LDS budget, more iterations than
+  // kBodyLoops -- and large levels of reduced storage keep the separate
+  // kernels too.
+  void setup_body() {
+    const char* e = std::getenv("ILBM_BODY_TILES");
+    const int nloop = ib_args().nloop;
+    if (c.dim != 2 || moving || cf || !stepbodyfn || n_ne == 0 || nloop > kBodyLoops || (e && e[0] == '0')) return;
+    if (c.n[0] > 0xffff || c.n[1] > 0x7fff) return;   // packed cells
+    if (st != 0 && ncells > kBodyReducedCells) return;
+    std::vector<int> where(band_cells, -1);   // list index of a band cell
+    for (int ci = 0; ci < n_ne; ++ci) where[ne_h[ci]] = ci;
+    auto list_cell = [&](const int p[2]) {
+      const int bi = p[0] - band_lo[0], bj = p[1] - band_lo[1];
+      return (bi < 0 || bi >= band_n[0] || bj < 0 || bj >= band_n[1]) ? -1 : where[(size_t)bj * band_n[0] + bi];
+    };
+    // stencil points of every marker: list index, or the ghost cell
+    struct Pt { int li; int p[2]; };
+    std::vector<Pt> st(25 * (size_t)nm);
+    for (int m = 0; m < nm; ++m)
+      for (int t = 0; t < 25; ++t) {
+        Pt& q = st[(size_t)m * 25 + t];
+        bool ghost = false;
+        int w[2];
+        for (int d = 0; d < 2; ++d) {
+          const int b = (int)std::floor((xm_h[(size_t)d * nm + m] - c.plo[d]) / c.dx[d]) - ioff[d];
+          const int p = b + (d == 0 ? t / 5 : t % 5) - 2;
+          if (p < -2 || p > c.n[d] + 1) return;
+          q.p[d] = w[d] = p;
+          if (p >= 0 && p <= c.n[d] - 1) continue;
+          if (c.periodic[d]) w[d] += (p < 0) ? c.n[d] : -c.n[d];
+          else ghost = true;
+        }
+        q.li = ghost ? -1 : list_cell(w);
+        if (!ghost && q.li < 0) return;
+      }
+    std::map<std::pair<int, int>, std::vector<int>> own;   // list cells of each tile
+    for (int ci = 0; ci < n_ne; ++ci)
+      own[{ne_h[ci] / band_n[0] / kBodyTile, ne_h[ci] % band_n[0] / kBodyTile}].push_back(ci);
+    std::vector<BodyTile> tiles;
+    std::vector<int> cells, rest, mk, pt, ep, em, esrc, gh;
+    std::vector<double> ghv;
+    std::vector<int> cslot(n_ne, -1), mslot(nm, -1);
+    std::vector<char> owned(nm, 0);
+    int lds = 0;
+    for (const auto& to : own) {
+      BodyTile T{};
+      std::vector<int> lc = to.second, lm;
+      std::fill(cslot.begin(), cslot.end(), -1);
+      std::fill(mslot.begin(), mslot.end(), -1);
+      for (size_t x = 0; x < lc.size(); ++x) cslot[lc[x]] = (int)x;
+      T.nown = (int)lc.size();
+      for (int it = nloop - 1; it >= 0; --it) {
+        // markers that reach the cells so far, then the cells of their stencils
+        const size_t c1 = lc.size(), m1 = lm.size();
+        for (size_t x = 0; x < c1; ++x)
+          for (int en = nee_h[lc[x]]; en < nee_h[n_ne + lc[x]]; ++en)
+            if (mslot[em_h[en]] < 0) { mslot[em_h[en]] = (int)lm.size(); lm.push_back(em_h[en]); }
+        for (size_t y = m1; y < lm.size(); ++y)
+          for (int t = 0; t < 25; ++t) {
+            const int li = st[(size_t)lm[y] * 25 + t].li;
+            if (li >= 0 && cslot[li] < 0) { cslot[li] = (int)lc.size(); lc.push_back(li); }
+          }
+        T.nmk[it] = (int)lm.size();
+        T.ncell[it] = (int)lc.size();
+      }
+      const int nc = (int)lc.size(), nmk = (int)lm.size();
+      T.cell0 = (int)rest.size(); T.mk0 = (int)mk.size(); T.pt0 = (int)pt.size();
+      T.gh0 = (int)gh.size(); T.ep0 = (int)ep.size(); T.ent0 = (int)em.size();
+      // own cells on the first wavefront, then a cell for each of the others' threads, then the rest
+      const size_t head = cells.size();
+      cells.resize(head + kBlock, band_lo[0] | band_lo[1] << 16);
+      for (int x = 0; x < nc; ++x) {
+        const int ij = (band_lo[0] + ne_h[lc[x]] % band_n[0]) | (band_lo[1] + ne_h[lc[x]] / band_n[0]) << 16;
+        if (x < T.nown) cells[head + x] = ij;
+        else if (x < T.nown + kBlock - kBodyOwn) cells[head + kBodyOwn + x - T.nown] = ij;
+        else rest.push_back(ij);
+      }
+      for (int y = 0; y < nmk; ++y) {
+        const bool mine = y < T.nmk[nloop - 1] && !owned[lm[y]];
+        if (mine) owned[lm[y]] = 1;
+        mk.push_back(lm[y] | (mine ? kMkOwner : 0));
+      }
+      std::map<std::pair<int, int>, int> gslot;
+      for (int t = 0; t < 25; ++t)
+        for (int y = 0; y < nmk; ++y) {
+          const Pt& q = st[(size_t)lm[y] * 25 + t];
+          if (q.li >= 0) { pt.push_back(cslot[q.li]); continue; }
+          auto ins = gslot.emplace(std::make_pair(q.p[0], q.p[1]), nc + T.ngh);
+          if (ins.second) {
+            const GhostSrc g0 = ghost_src(q.p);
+            const int li = (g0.kind == 1) ? lc[0] : list_cell(g0.cell);
+            if (li < 0 || cslot[li] < 0) return;   // its source is not among the tile's cells
+            gh.push_back(cslot[li] | g0.kind << 16);
+            ghv.push_back(g0.v[0]);
+            ghv.push_back(g0.v[1]);
+            ++T.ngh;
+          }
+          pt.push_back(ins.first->second);
+        }
+      T.necell = (nloop > 1) ? T.ncell[1] : T.nown;
+      for (int x = 0; x < T.necell; ++x) {
+        ep.push_back(T.nent);
+        for (int en = nee_h[lc[x]]; en < nee_h[n_ne + lc[x]]; ++en, ++T.nent) {
+          em.push_back(mslot[em_h[en]] | (ec_h[en] >> 9) << 16);
+          esrc.push_back(en);
+        }
+      }
+      ep.push_back(T.nent);
+      if (nc + T.ngh > 0xffff || nmk > 0xffff) return;
+      lds = std::max(lds, body_tile_lds(T));
+      tiles.push_back(T);
+    }
+    for (BodyTile& T : tiles) T.cell0 += (int)cells.size();
+    cells.insert(cells.end(), rest.begin(), rest.end());
+    lds = std::max(lds, (int)(64 * ((band_cells + 255) / 256)));   // the record's wave sums
+    if (lds > kBodyLds) return;
+    std::vector<unsigned char> mask(band_cells, 0);
+    for (int b : ne_h) mask[b] = 1;
+    std::vector<int> ints;
+    size_t off[6];
+    const std::vector<int>* parts[6] = {&cells, &mk, &pt, &ep, &em, &gh};
+    for (int x = 0; x < 6; ++x) {
+      off[x] = ints.size();
+      ints.insert(ints.end(), parts[x]->begin(), parts[x]->end());
+    }
+    const size_t osrc = ints.size();
+    ints.insert(ints.end(), esrc.begin(), esrc.end());
+    body_mask = dev_alloc<unsigned char>(band_cells);
+    body_int = dev_alloc<int>(ints.size());
+    body_dbl = dev_alloc<double>(em.size() + ghv.size());
+    body_tiles = dev_alloc<BodyTile>(tiles.size());
+    HIPCHK(hipMemcpyAsync(body_mask, mask.data(), mask.size(), hipMemcpyHostToDevice, stream));
+    HIPCHK(hipMemcpyAsync(body_int, ints.data(), sizeof(int) * ints.size(), hipMemcpyHostToDevice, stream));
+    HIPCHK(hipMemcpyAsync(body_tiles, tiles.data(), sizeof(BodyTile) * tiles.size(), hipMemcpyHostToDevice, stream));
+    if (!ghv.empty())
+      HIPCHK(hipMemcpyAsync(body_dbl + em.size(), ghv.data(), sizeof(double) * ghv.size(), hipMemcpyHostToDevice,
+                            stream));
+    // the entries' weights, in the tiles' order
+    hipLaunchKernelGGL(k_gather_doubles, dim3((unsigned)((em.size() + 255) / 256)), dim3(256), 0, stream,
+                       (const double*)entw_d, (const int*)(body_int + osrc), body_dbl, (int64_t)em.size());
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(stream));   // host vectors go out of scope
+    body.tiles = body_tiles;
+    body.ntile = (int)tiles.size();
+    body.cells = body_int + off[0]; body.mk = body_int + off[1]; body.pt = body_int + off[2];
+    body.eptr = body_int + off[3]; body.em = body_int + off[4]; body.gh = body_int + off[5];
+    body.ew = body_dbl;
+    body.ghv = body_dbl + em.size();
+    body.lds = lds;
+    body_ok = true;
+  }
+
+  // slot 0: the arrays the getters and the checkpoint read
+  BodyArgs body_args(int slot) const {
+    BodyArgs B = body;
+    B.ib = ib_args();
+    if (slot) { B.ib.F = body_F; B.ib.Fband = body_Fband; }
+    return B;
+  }
+
+  // nsteps steps of a level with body tiles: the forcing of the first step
+  // alone, then one launch per step (plus the ghost slabs where the
+  // stream-collide kernel does not write them, and an IVC body's solve) with
+  // the next step's forcing in its first blocks.  Step s uses slot
+  // (nsteps - 1 - s) & 1, so the last one leaves its force in slot 0.
+  void advance_body(int nsteps, bool want_state) {
+    if (!body_F) {
+      body_F = dev_alloc<double>(3 * (size_t)nm * ib_args().nloop);
+      body_Fband = dev_alloc<double>(3 * band_cells);
+    }
+    const int64_t npad = wrap ? 0 : slabs.face_off[slabs.nface];
+    BodyArgs B[2] = {body_args(0), body_args(1)};
+    const bool ivc = B[0].ib.use_ivc != 0;
+    bodyfn(1, stream, B[(nsteps - 1) & 1], body_mask, g, gbuf[cur], tau);
+    for (int s = 0; s < nsteps; ++s) {
+      const double time = t_new;
+      t_old = t_new;
+      t_new += dt;
+      const bool last = s == nsteps - 1;
+      const BodyArgs& now = B[(nsteps - 1 - s) & 1];
+      const BodyArgs& next = B[(nsteps - s) & 1];
+      if (ivc) bodyfn(2, stream, now, body_mask, g, gbuf[cur], tau);
+      if (npad && !slabs_fresh)
+        ghostfn(dim3((unsigned)((npad + kGhostBlock - 1) / kGhostBlock)), dim3(kGhostBlock), stream, ghost_args());
+      StepArgs sa = step_args(want_state && last);
+      sa.body_mask = body_mask;
+      sa.Fband = now.ib.Fband;
+      sa.Fnext = last ? nullptr : next.ib.Fband;
+      sa.dt = dt;
+      sa.partial = mring + (int64_t)mring_used * nblocks;
+      stepbodyfn(grid, block, stream, sa, now.ib, rec_args(time, s), next, !last);
+      ring_step(stream, s, !last, false);
+      slabs_fresh = gfuse;
+      cur ^= 1;
+      ++istep;
+      HIPCHK(hipGetLastError());
+    }
   }
 
   // positions, spreading lists and (for IVC) the inverse operator
@@ -1000,6 +1310,10 @@ struct Level {
       HIPCHK(hipMemcpyAsync(entc_d, ec.data(), sizeof(int) * nent, hipMemcpyHostToDevice, stream));
     }
     HIPCHK(hipStreamSynchronize(stream));  // host vectors go out of scope
+    ne_h = std::move(ne);
+    nee_h = std::move(nee);
+    em_h = std::move(em);
+    ec_h = std::move(ec);
   }
 
   // build_ivc_operator + lu_factorize (IBMarkerDF.cpp:1081-1142); the solve
@@ -1130,6 +1444,19 @@ struct Level {
     return mv;
   }
 
+  // the force record of the step from `time`, row `row` of the history
+  RecArgs rec_args(double time, int row) const {
+    RecArgs r{};
+    r.partial = (ring_slot >= 0) ? fp_ring[ring_slot] : fpartial; r.sums = sums_d; r.state = frstate_d;
+    r.hist = force_dev; r.row = row; r.ncol = ncol; r.method = c.force_eval_method;
+    r.time = time + dt; r.step = (double)(istep + 1);
+    r.dV = (c.dim == 3) ? c.dx[0] * c.dx[1] * c.dx[2] : c.dx[0] * c.dx[1];
+    r.U0 = c.U0; r.R = c.R;
+    r.clock = nullptr;
+    if (rec_override) { r.time = rec_time; r.step = rec_step; }
+    return r;
+  }
+
   // IBMarkerDF::update_forcing (IBMarkerDF.cpp:1522-1917) on the band, ending
   // with the export of F fused with the Guo term of the coming collision and
   // with the ComputeIBForce record of the step (row `row` of the history).
@@ -1171,14 +1498,7 @@ struct Level {
       hipLaunchKernelGGL(k_ib_sums, dim3(1), dim3(kSumsBlock), 0, stream, a);
       if (!a.ev_from_macro) hipLaunchKernelGGL(k_ib_correct, dim3(gb), dim3(tb), 0, stream, a);
     }
-    RecArgs r{};
-    r.partial = (ring_slot >= 0) ? fp_ring[ring_slot] : fpartial; r.sums = sums_d; r.state = frstate_d;
-    r.hist = force_dev; r.row = row; r.ncol = ncol; r.method = c.force_eval_method;
-    r.time = time + dt; r.step = (double)(istep + 1);
-    r.dV = (c.dim == 3) ? c.dx[0] * c.dx[1] * c.dx[2] : c.dx[0] * c.dx[1];
-    r.U0 = c.U0; r.R = c.R;
-    r.clock = nullptr;
-    if (rec_override) { r.time = rec_time; r.step = rec_step; }
+    const RecArgs r = rec_args(time, row);
     const int mode = fix_mode();
     const unsigned gfix = fix_blocks();
     if (gfix) fixfn(mode, dim3(gfix), dim3(tb), stream, a, g, gbuf[cur], tau, r);
@@ -1438,7 +1758,7 @@ struct Level {
   // the near box (IB band grown by one cell; the whole extent of a periodic
   // dimension it would wrap across) and the resources of the overlapped step
   bool split_ready() {
-    if (!overlap || timing || !ib || cf || window || band_cells <= 0) return false;
+    if (!overlap || timing || !ib || cf || window || band_cells <= 0 || body_ok) return false;
     // below ~1M cells the two cross-stream waits per step cost more than
     // the overlap saves (512x256 D2Q9 FP64: 2.5 -> 1.9 GLUPS with it)
     if (ncells < ((int64_t)1 << 20)) return false;
@@ -1503,10 +1823,8 @@ struct Level {
         F_ring[0] = F_d;
         fp_ring[0] = fpartial;
         for (int k = 0; k < kRecRing; ++k) {
-          if (k > 0) {
-            F_ring[k] = dev_alloc<double>(3 * nm);
-            fp_ring[k] = dev_alloc<double>(fpartial_n);
-          }
+          if (k > 0 && !F_ring[k]) F_ring[k] = dev_alloc<double>(3 * nm);
+          if (k > 0 && !fp_ring[k]) fp_ring[k] = dev_alloc<double>(fpartial_n);
         }
       }
     }
@@ -1829,7 +2147,9 @@ struct Level {
       }
     }
     state_valid = false;
-    for (int s = 0; s < nsteps; ++s) {
+    const bool body = body_ok && !timing;
+    if (body) advance_body(nsteps, want_state);
+    for (int s = 0; s < nsteps && !body; ++s) {
       const double time = t_new;  // timeStepWithSubcycling, AmrCoreLBM.cpp:1730-1733
       t_old = t_new;
       t_new += dt;
