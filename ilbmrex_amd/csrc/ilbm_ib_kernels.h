@@ -819,7 +819,8 @@ constexpr int kSumsBlock = 256;
 // Thread index and count of a block in linear order (x fastest), so that the
 // reductions below form the same wavefronts and trees in a block of
 // kSumsBlock x 1 threads and in one of the stream-collide kernel's 2D shapes.
-// Of a larger block the first kSumsBlock threads reduce.
+// (A step's launch may also hold fewer threads: rows 129 to 192 cells wide
+// are blocks of 192.)
 __device__ inline int lin_tid() { return (int)(threadIdx.x + threadIdx.y * blockDim.x); }
 __device__ inline int lin_nt() { return (int)(blockDim.x * blockDim.y); }
 
@@ -827,11 +828,10 @@ __device__ inline int lin_nt() { return (int)(blockDim.x * blockDim.y); }
 __device__ __forceinline__ void sums_body(const IbArgs& a, const double* F, int first_iter) {
   __shared__ double lds[6][16];
   const int nm = a.nm;
-  const int t = lin_tid();
-  constexpr int nt = kSumsBlock;
+  const int t = lin_tid(), nt = lin_nt();
   double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   const double z0 = (a.dim == 3) ? a.z0 : 0.0;
-  for (int m = t; m < nm && t < nt; m += nt) {
+  for (int m = t; m < nm; m += nt) {
     const double fx = F[m] * a.dv, fy = F[nm + m] * a.dv, fz = F[2 * nm + m] * a.dv;
     const double rx = a.xm[m] - a.x0, ry = a.xm[nm + m] - a.y0;
     const double rz = (a.dim == 3) ? a.xm[2 * nm + m] - z0 : 0.0;
@@ -842,12 +842,12 @@ __device__ __forceinline__ void sums_body(const IbArgs& a, const double* F, int 
   }
   for (int c = 0; c < 6; ++c) {
     const double r = wave_sum(acc[c]);
-    if ((t & 63) == 0 && t < nt) lds[c][t >> 6] = r;
+    if ((t & 63) == 0) lds[c][t >> 6] = r;
   }
   __syncthreads();
   if (t < 6) {
     double s = 0.0;
-    for (int wv = 0; wv < nt / 64; ++wv) s += lds[t][wv];
+    for (int wv = 0; wv < (nt + 63) / 64; ++wv) s += lds[t][wv];
     if (t < 3) a.sums[t] = first_iter ? s : a.sums[t] + s;
     else a.sums[t] = s;
   }
@@ -1437,20 +1437,19 @@ __device__ __forceinline__ void sums_record_body(const IbArgs& a, const RecArgs&
   __shared__ double lds[3][16];
   sums_body(a, a.F, 1);
   __syncthreads();
-  const int tid = lin_tid();
-  constexpr int nt = kSumsBlock;
+  const int tid = lin_tid(), nt = lin_nt();
   double acc[3] = {0.0, 0.0, 0.0};
-  for (int t = tid; t < nblk && tid < nt; t += nt)
+  for (int t = tid; t < nblk; t += nt)
     for (int c = 0; c < 3; ++c) acc[c] += rec.partial[(int64_t)c * nblk + t];
   for (int c = 0; c < 3; ++c) {
     const double r = wave_sum(acc[c]);
-    if ((tid & 63) == 0 && tid < nt) lds[c][tid >> 6] = r;
+    if ((tid & 63) == 0) lds[c][tid >> 6] = r;
   }
   __syncthreads();
   if (tid == 0) {
     double sum[3] = {0.0, 0.0, 0.0};
     for (int c = 0; c < 3; ++c)
-      for (int wv = 0; wv < nt / 64; ++wv) sum[c] += lds[c][wv];
+      for (int wv = 0; wv < (nt + 63) / 64; ++wv) sum[c] += lds[c][wv];
     write_force_record(a, rec, sum);
   }
 }

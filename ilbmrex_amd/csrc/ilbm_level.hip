@@ -527,7 +527,8 @@ struct Level {
   BodyFn bodyfn = nullptr;
   // body tiles (see body_tile): their tables, the mask of their cells in the
   // band, and the second slot of force and export
-  bool body_ok = false;
+  // (built when the level first steps on its own; a batch's cases never do)
+  bool body_ok = false, body_tried = false;
   unsigned char* body_mask = nullptr;
   int* body_int = nullptr;
   double* body_dbl = nullptr;
@@ -970,7 +971,6 @@ struct Level {
     fpartial_n = 3 * ((band_cells + 255) / 256 + band_cells / kSpreadWaves + tiles + 2);
     fpartial = dev_alloc<double>(fpartial_n);
     upload_markers();
-    setup_body();
     ncol = (c.dim == 3) ? 33 : 23;
   }
 
@@ -1022,6 +1022,7 @@ struct Level {
   // kBodyLoops -- and large levels of reduced storage keep the separate
   // kernels too.
   void setup_body() {
+    body_tried = true;
     const char* e = std::getenv("ILBM_BODY_TILES");
     const int nloop = ib_args().nloop;
     if (c.dim != 2 || moving || cf || !stepbodyfn || n_ne == 0 || nloop > kBodyLoops || (e && e[0] == '0')) return;
@@ -2130,6 +2131,7 @@ struct Level {
     if (nsteps == 0) return;
     if (want_state) ensure_exports();
     grow_histories(nsteps, nsteps);
+    if (ib && !body_tried) setup_body();
     const bool split = split_ready();
     ensure_mring(split);
     if (split) {

@@ -77,3 +77,23 @@ def test_body_tiles_equal_separate_kernels_when_diverging(monkeypatch, storage):
     assert not np.isfinite(ref["history"]).all()
     for k, v in ref.items():
         assert np.array_equal(one[k], v, equal_nan=True), k
+
+
+def test_record_beside_a_step_of_192_thread_blocks():
+    """The force record rides in the stream-collide launch of a hierarchy's
+    finest level, whose blocks hold 192 threads when its box is 129 to 192
+    cells wide; more markers than that."""
+    import refcpu
+    from ilbmrex_amd.native import AmrHierarchy
+    c = cf.cylinder_2d(nx=110, ny=56, D=12.0, xc=50.0, yc=28.0, U=0.05, Re=60.0).replace(n_marker=230)
+    boxes = [((20, 20, 0), (179, 91, 0))]
+    print("[body] hierarchy with a finest level 160 cells wide", flush=True)
+    state = (1.0, 0.05, 0.0, 0.0)
+    with AmrHierarchy(c, boxes, 2, state) as h:
+        h.advance(3, want_state=True)
+        o = refcpu.AmrOracle(c, boxes, 2, cf.uniform_init(c, u=(0.05, 0.0, 0.0)))
+        o.advance(3)
+        assert np.array_equal(h.macro(1), o.macro(1))
+        rec, got = o.force_record(), h.force_history()[-1]
+    floor = 1e-10 * np.abs(rec).max()
+    assert np.all(np.abs(got - rec) <= 1e-12 * np.abs(rec) + floor), (got, rec)
