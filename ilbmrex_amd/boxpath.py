@@ -4,19 +4,22 @@ BoxLevel keeps the reference's own state on the device -- f_new / f_old
 (ndir components) and macro_new / macro_old (nmac components: rho, ux, uy,
 uz, vorticity, pressure), AMReX Array4 layout with 3 ghost cells
 (AmrCoreLBM.H:175-180, 276) -- in buffers of the library's allocator, and
-steps it with one ilbm_box_* / ilbm_ib_* call per stage in the order of
-Source/Core/AdvanceLBMAtLevel.cpp:20-386 for a level of one box:
+steps it with ilbm_box_* / ilbm_ib_* calls in the order of
+Source/Core/AdvanceLBMAtLevel.cpp:20-386 for a level of one box, with the
+calls that run several stages in one pass over the arrays:
 
     swap f_new/f_old, macro_new/macro_old
-    FillPatch(f_old) -> sfSborder       copy + periodic images + mesoscopicBcFill
-                                        (lev > 0: equilibrium of the coarse
-                                        interpolation in the ghost cells)
-    FillPatch(macro_old) -> smSborder   copy + periodic images + macroBcFill
-                                        (lev > 0: cell_cons_interp of the coarse)
+    FillPatch(macro_old) -> smSborder   ilbm_box_fill_patch: valid cells,
+                                        periodic images, macroBcFill (lev > 0:
+                                        ilbm_box_cf_fill_patch, cell_cons_interp
+                                        of the coarse; it also fills the ghost
+                                        cells of sfSborder with the
+                                        interpolation's equilibrium)
     force scratch: prescribed force or 0; IBMarkerDF::update_forcing on the
                    aliases rho, u, v, w of smSborder; FillBoundary
-    collide(sfSborder; smSborder, force)
-    FillBoundary(sfSborder), bounce-back ghosts
+    FillPatch(f_old) -> sfSborder, collide(sfSborder; smSborder, force),
+    FillBoundary(sfSborder)             ilbm_box_fill_collide
+    bounce-back ghosts
     stream + forced macros -> f_new, macro_new
 
 Sum(Rho) and ComputeIBForce (AmrCoreLBM.cpp:366-414, 456-701) are composed
@@ -67,6 +70,7 @@ class _Arr:
         self.strides = (js, ks, ns) if pad else (0, 0, 0)
         self.js, self.ks, self.ns = js, ks, ns
         self.dev = native.DeviceArray((ncomp * ns,))
+        self._refs = {}
         native._check(native.load().ilbm_box_setval(self.ref(), 0.0, None), "ilbm_box_setval")
 
     def fab(self, comp=0, ncomp=None):
@@ -74,7 +78,11 @@ class _Arr:
                                self.strides, comp)
 
     def ref(self, comp=0, ncomp=None):
-        return C.byref(self.fab(comp, ncomp))
+        # the array's memory and box do not change: one descriptor per alias
+        r = self._refs.get((comp, ncomp))
+        if r is None:
+            r = self._refs[(comp, ncomp)] = C.byref(self.fab(comp, ncomp))
+        return r
 
     def _view(self, flat):
         return np.lib.stride_tricks.as_strided(flat, shape=(self.ncomp, self.n[2], self.n[1], self.n[0]),
@@ -129,6 +137,9 @@ class BoxLevel:
             native._check(self.L.ilbm_ib_create(C.byref(self.desc), _i3(self.vlo), _i3(self.vhi), C.byref(h)),
                           "ilbm_ib_create")
             self.ib = h
+        self._d, self._lo, self._hi = C.byref(self.desc), _i3(self.vlo), _i3(self.vhi)
+        self._patch = None     # update_derived's macros with one ghost layer
+        self._work = None      # workspace of the force sums
         self.have_prev = False
         self.prev_body = (0.0, 0.0, 0.0)
         self.record = None
@@ -151,7 +162,7 @@ class BoxLevel:
 
     def equilibrium(self):
         """InitEquilibrium: f_new = f_old = feq(macro_new) on the valid box."""
-        d = C.byref(self.desc)
+        d = self._d
         self._check(self.L.ilbm_box_equilibrium(d, self.m_new.ref(), self.f_new.ref(), _i3(self.vlo), _i3(self.vhi),
                                                 None), "box_equilibrium")
         self._check(self.L.ilbm_box_copy(self.f_new.ref(), self.f_old.ref(), _i3(self.vlo), _i3(self.vhi), self.q,
@@ -161,60 +172,61 @@ class BoxLevel:
         if self.ib:
             self.L.ilbm_ib_destroy(self.ib)
             self.ib = None
-        for a in (self.f_new, self.f_old, self.sfS, self.m_new, self.m_old, self.smS, self.fx):
-            a.free()
+        for a in (self.f_new, self.f_old, self.sfS, self.m_new, self.m_old, self.smS, self.fx, self._patch, self._work):
+            if a is not None:
+                a.free()
 
     # -- FillPatch ---------------------------------------------------------
-    def _fill_patch_single(self, dst: _Arr, src: _Arr, meso: bool):
-        d = C.byref(self.desc)
-        nc = dst.ncomp
-        self._check(self.L.ilbm_box_setval(dst.ref(), 0.0, None), "box_setval")
-        self._check(self.L.ilbm_box_copy(src.ref(), dst.ref(), _i3(self.vlo), _i3(self.vhi), nc, None),
-                    "box_copy")                                              # ParallelCopy
-        self._check(self.L.ilbm_box_fill_periodic(d, dst.ref(), _i3(self.vlo), _i3(self.vhi), None),
-                    "box_fill_periodic")
-        self._check(self.L.ilbm_box_fill_physical(d, dst.ref(), int(meso), None), "box_fill_physical")
-
     def fill_patch(self, time, coarse: Optional["BoxLevel"] = None):
-        """sfSborder / smSborder of a step starting at `time`."""
+        """sfSborder / smSborder of a step starting at `time`, before the
+        collision (advance_level collides in the same pass)."""
+        L, d, lo, hi = self.L, self._d, self._lo, self._hi
         if coarse is None:
-            self._fill_patch_single(self.sfS, self.f_old, True)
-            self._fill_patch_single(self.smS, self.m_old, False)
+            self._check(L.ilbm_box_fill_patch(d, self.f_old.ref(), self.sfS.ref(), 1, lo, hi, None), "box_fill_patch")
+            self._check(L.ilbm_box_fill_patch(d, self.m_old.ref(), self.smS.ref(), 0, lo, hi, None), "box_fill_patch")
             return
-        # FillPatchMacro / FillPatchMesoscopic for lev > 0: own valid cells,
-        # ghosts from the coarse level at `time`
-        for dst, src, nc in ((self.smS, self.m_old, self.nmac), (self.sfS, self.f_old, self.q)):
-            self._check(self.L.ilbm_box_copy(src.ref(), dst.ref(), _i3(self.vlo), _i3(self.vhi), nc, None),
-                        "box_copy")
-        self._check(self.L.ilbm_box_cf_fill(C.byref(self.desc), coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old,
-                                            coarse.t_new, time, self.sfS.ref(), self.smS.ref(), self.nmac,
-                                            _i3(self.vlo), _i3(self.vhi), None), "box_cf_fill")
+        self._check(L.ilbm_box_copy(self.f_old.ref(), self.sfS.ref(), lo, hi, self.q, None), "box_copy")
+        self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
+                                             time, self.sfS.ref(), self.smS.ref(), self.m_old.ref(), self.nmac,
+                                             lo, hi, None), "box_cf_fill_patch")
 
     # -- one AdvancePhiAtLevel ------------------------------------------------
     def advance_level(self, time, coarse: Optional["BoxLevel"] = None):
         self.f_new, self.f_old = self.f_old, self.f_new
         self.m_new, self.m_old = self.m_old, self.m_new
-        self.fill_patch(time, coarse)
-        d = C.byref(self.desc)
-        lo, hi = _i3(self.vlo), _i3(self.vhi)
+        L, d, lo, hi = self.L, self._d, self._lo, self._hi
+        if coarse is None:
+            self._check(L.ilbm_box_fill_patch(d, self.m_old.ref(), self.smS.ref(), 0, lo, hi, None), "box_fill_patch")
+        else:
+            # FillPatchMacro / FillPatchMesoscopic for lev > 0: own valid
+            # cells, ghosts from the coarse level at `time`
+            self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
+                                                 time, self.sfS.ref(), self.smS.ref(), self.m_old.ref(), self.nmac,
+                                                 lo, hi, None), "box_cf_fill_patch")
         force = None
         if self.has_force:
-            for c in range(3):
-                self._check(self.L.ilbm_box_setval(self.fx.ref(c, 1), float(self.uniform_force[c]), None),
-                            "box_setval")
+            u = self.uniform_force
+            if u[0] == u[1] == u[2]:
+                self._check(L.ilbm_box_setval(self.fx.ref(), float(u[0]), None), "box_setval")
+            else:
+                for c in range(3):
+                    self._check(L.ilbm_box_setval(self.fx.ref(c, 1), float(u[c]), None), "box_setval")
             if self.ib:
-                s = self.smS
-                self._check(self.L.ilbm_ib_update_forcing(
-                    self.ib, s.ref(0, 1), s.ref(1, 1), s.ref(2, 1), s.ref(3, 1),
-                    self.fx.ref(0, 1), self.fx.ref(1, 1), self.fx.ref(2, 1), self.dt, time, None), "ib_update_forcing")
-            self._check(self.L.ilbm_box_fill_periodic(d, self.fx.ref(), lo, hi, None), "box_fill_periodic")
+                s, fx = self.smS, self.fx
+                self._check(L.ilbm_ib_update_forcing(self.ib, s.ref(0, 1), s.ref(1, 1), s.ref(2, 1), s.ref(3, 1),
+                                                     fx.ref(0, 1), fx.ref(1, 1), fx.ref(2, 1), self.dt, time, None),
+                            "ib_update_forcing")
+            self._check(L.ilbm_box_fill_periodic(d, self.fx.ref(), lo, hi, None), "box_fill_periodic")
             force = self.fx.ref()
-        self._check(self.L.ilbm_box_collide(d, self.sfS.ref(), self.smS.ref(), force, lo, hi, None), "box_collide")
-        self._check(self.L.ilbm_box_fill_periodic(d, self.sfS.ref(), lo, hi, None), "box_fill_periodic")
-        self._check(self.L.ilbm_box_bounce_back(d, self.sfS.ref(), lo, hi, None), "box_bounce_back")
-        force = self.fx.ref() if self.has_force else None
-        self._check(self.L.ilbm_box_stream_macro(d, self.sfS.ref(), self.f_new.ref(), self.m_new.ref(), force, lo, hi,
-                                                 None), "box_stream_macro")
+        self._check(L.ilbm_box_fill_collide(d, self.f_old.ref(), self.sfS.ref(), self.smS.ref(), force,
+                                            int(coarse is None), lo, hi, None), "box_fill_collide")
+        if coarse is not None:
+            # FillBoundary of the collided level (a refined box keeps its
+            # ghost cells inside the domain: nothing periodic to fill)
+            self._check(L.ilbm_box_fill_periodic(d, self.sfS.ref(), lo, hi, None), "box_fill_periodic")
+        self._check(L.ilbm_box_bounce_back(d, self.sfS.ref(), lo, hi, None), "box_bounce_back")
+        self._check(L.ilbm_box_stream_macro(d, self.sfS.ref(), self.f_new.ref(), self.m_new.ref(), force, lo, hi,
+                                            None), "box_stream_macro")
 
     def step(self):
         """timeStepWithSubcycling at max_level = 0, then ComputeIBForce."""
@@ -242,7 +254,14 @@ class BoxLevel:
         -sum(F dv), time-centred body force, coefficients."""
         c = self.case
         dV = c.dx[0] * c.dx[1] * (c.dx[2] if self.dim == 3 else 1.0)
-        s = [self.box_sum(self.fx, k) for k in range(3)]
+        if self._work is None:
+            n = C.c_int64(0)
+            self._check(self.L.ilbm_box_sums_workspace(self._lo, self._hi, 3, C.byref(n)), "box_sums_workspace")
+            self._work = native.DeviceArray((n.value // 8,))
+        sums = (C.c_double * 3)()
+        self._check(self.L.ilbm_box_sums(self.fx.ref(), 0, 3, self._lo, self._hi, self._work.ptr, self._work.nbytes,
+                                         sums, None), "box_sums")
+        s = list(sums)
         if self.dim != 3:
             s[2] = 0.0
         eul = tuple(-(x * dV) / self.dt for x in s)
@@ -300,24 +319,19 @@ class BoxLevel:
         """UpdateDerivedMacroFields (AmrCoreLBM.cpp:150-168): FillPatchMacro
         of comps 0..3 with one ghost at `time` (the level's macro_new), then
         vorticity and pressure into comps 4, 5 of macro_new."""
-        g = [1 if d < self.dim else 0 for d in range(3)]
-        plo = tuple(self.vlo[d] - g[d] for d in range(3))
-        phi = tuple(self.vhi[d] + g[d] for d in range(3))
-        patch = _Arr(4, plo, phi, False)
-        self._check(self.L.ilbm_box_copy(self.m_new.ref(0, 4), patch.ref(), _i3(self.vlo), _i3(self.vhi), 4, None),
-                    "box_copy")
+        if self._patch is None:
+            g = [1 if d < self.dim else 0 for d in range(3)]
+            self._patch = _Arr(4, tuple(self.vlo[d] - g[d] for d in range(3)),
+                               tuple(self.vhi[d] + g[d] for d in range(3)), False)
+        L, d, lo, hi, patch = self.L, self._d, self._lo, self._hi, self._patch
         if coarse is None:
-            self._check(self.L.ilbm_box_fill_periodic(C.byref(self.desc), patch.ref(), _i3(self.vlo), _i3(self.vhi),
-                                                      None), "box_fill_periodic")
-            self._check(self.L.ilbm_box_fill_physical(C.byref(self.desc), patch.ref(), 0, None), "box_fill_physical")
+            self._check(L.ilbm_box_fill_patch(d, self.m_new.ref(0, 4), patch.ref(), 0, lo, hi, None), "box_fill_patch")
         else:
-            self._check(self.L.ilbm_box_cf_fill(C.byref(self.desc), coarse.m_old.ref(), coarse.m_new.ref(),
-                                                coarse.t_old, coarse.t_new, time, None, patch.ref(), 4,
-                                                _i3(self.vlo), _i3(self.vhi), None), "box_cf_fill")
+            self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
+                                                 time, None, patch.ref(), self.m_new.ref(0, 4), 4, lo, hi, None),
+                        "box_cf_fill_patch")
         dst = target if target is not None else self.m_new
-        self._check(self.L.ilbm_box_derived(C.byref(self.desc), patch.ref(), dst.ref(), _i3(self.vlo), _i3(self.vhi),
-                                            None), "box_derived")
-        patch.free()
+        self._check(L.ilbm_box_derived(d, patch.ref(), dst.ref(), lo, hi, None), "box_derived")
 
 
 class BoxHierarchy:

@@ -370,17 +370,16 @@ struct Amr {
     for (int d = 0; d < 3; ++d) { F.lo[d] = P.lo[d]; F.hi[d] = P.hi[d]; }
     F.js = P.js; F.ks = P.ks; F.ns = P.ns; F.cells = P.ns; F.nc = 4;
     const int64_t cells = V.ncells;
-    hipLaunchKernelGGL(k_fab_from_cells, grid_for(cells), dim3(256), 0, stream, F, (const double*)V.mout, V.c.n[0],
-                       V.c.n[1], cells);
     if (l == 0) {
       const BoxGeom G = box_geom(V.c, nullptr, nullptr);
-      hipLaunchKernelGGL(k_box_fill_periodic, grid_for(P.ns), dim3(256), 0, stream, F, G);
+      const Fab S = cells_fab(V.mout, V.c, 4);
       with_lattice(V.lat, [&](auto lat) {
         using LAT = decltype(lat);
-        for (int pass = 1; pass <= dim; ++pass)
-          hipLaunchKernelGGL(k_box_fill_physical<LAT>, grid_for(P.ns), dim3(256), 0, stream, F, G, pass, 0);
+        launch_fill_patch<LAT>(S, F, G, 0, stream);
       });
     } else {
+      hipLaunchKernelGGL(k_fab_from_cells, grid_for(cells), dim3(256), 0, stream, F, (const double*)V.mout, V.c.n[0],
+                         V.c.n[1], cells);
       PatchCfArgs a{};
       a.P = P;
       for (int d = 0; d < 3; ++d) { a.n[d] = V.c.n[d]; a.ioff[d] = (d < dim) ? V.ioff[d] : 0; }

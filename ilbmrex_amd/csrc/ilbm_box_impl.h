@@ -24,6 +24,9 @@ struct Fab {
   __host__ __device__ double& at(int i, int j, int k, int n) const {
     return p[(int64_t)(i - lo[0]) + (int64_t)(j - lo[1]) * js + (int64_t)(k - lo[2]) * ks + (int64_t)n * ns];
   }
+  __host__ __device__ int64_t off(int i, int j, int k) const {
+    return (int64_t)(i - lo[0]) + (int64_t)(j - lo[1]) * js + (int64_t)(k - lo[2]) * ks;
+  }
   __host__ __device__ bool contains(int i, int j, int k) const {
     return i >= lo[0] && i <= hi[0] && j >= lo[1] && j <= hi[1] && k >= lo[2] && k <= hi[2];
   }
@@ -63,17 +66,98 @@ struct BoxGeom {
 
 __device__ inline int nonper_out_cnt(const BoxGeom& G, const int iv[3]) {
   int c = 0;
-  for (int d = 0; d < G.dim; ++d)
-    if (!G.periodic[d] && (iv[d] < 0 || iv[d] > G.n[d] - 1)) ++c;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (d < G.dim && !G.periodic[d] && (iv[d] < 0 || iv[d] > G.n[d] - 1)) ++c;
   return c;
+}
+
+// Cells of a fab outside a box, in up to six slabs: below and above it in z
+// (whole planes), then in y (whole rows), then in x.  A thread per ghost
+// cell: the fills of a level's ghost layers touch nothing else (a 134x102x102
+// fab around 128x96x96 cells has 15 % ghost cells).
+struct GhostBox {
+  int lo[6][3], n[6][3];
+  int64_t off[7];         // prefix sums; off[6]: the number of ghost cells
+};
+
+static GhostBox ghost_box(const Fab& F, const int blo[3], const int bhi[3]) {
+  GhostBox g{};
+  int lo[3], hi[3];
+  for (int d = 0; d < 3; ++d) { lo[d] = F.lo[d]; hi[d] = F.hi[d]; }
+  int64_t off = 0;
+  int s = 0;
+  for (int d = 2; d >= 0; --d) {
+    for (int side = 0; side < 2; ++side, ++s) {
+      int64_t cnt = 1;
+      for (int e = 0; e < 3; ++e) { g.lo[s][e] = lo[e]; g.n[s][e] = hi[e] - lo[e] + 1; }
+      if (side == 0) g.n[s][d] = std::max(0, std::min(blo[d], hi[d] + 1) - lo[d]);
+      else { g.lo[s][d] = std::max(bhi[d] + 1, lo[d]); g.n[s][d] = std::max(0, hi[d] - g.lo[s][d] + 1); }
+      for (int e = 0; e < 3; ++e) cnt *= g.n[s][e];
+      g.off[s] = off;
+      off += cnt;
+    }
+    lo[d] = std::max(lo[d], blo[d]);
+    hi[d] = std::min(hi[d], bhi[d]);
+    if (hi[d] < lo[d]) {   // the box and the fab do not meet: every cell is in this pair of slabs
+      for (; s < 6; ++s) { g.off[s] = off; for (int e = 0; e < 3; ++e) { g.lo[s][e] = 0; g.n[s][e] = 0; } }
+      break;
+    }
+  }
+  g.off[6] = off;
+  return g;
+}
+
+// cell t (x fastest) of a box, with 32-bit divisions where its count allows
+__device__ inline void box_cell(const int lo[3], int nx, int ny, int64_t cells, int64_t t, int iv[3]) {
+  if (cells < ((int64_t)1 << 32)) {
+    const uint32_t u = (uint32_t)t, row = u / (uint32_t)nx, pl = row / (uint32_t)ny;
+    iv[0] = lo[0] + (int)(u - row * (uint32_t)nx);
+    iv[1] = lo[1] + (int)(row - pl * (uint32_t)ny);
+    iv[2] = lo[2] + (int)pl;
+  } else {
+    iv[0] = lo[0] + (int)(t % nx);
+    iv[1] = lo[1] + (int)((t / nx) % ny);
+    iv[2] = lo[2] + (int)(t / ((int64_t)nx * ny));
+  }
+}
+
+// (scalar selects: an array copied under a condition would be indexed in
+// scratch memory)
+__device__ inline void ghost_cell(const GhostBox& g, int64_t t, int iv[3]) {
+  int lx = g.lo[0][0], ly = g.lo[0][1], lz = g.lo[0][2], nx = g.n[0][0], ny = g.n[0][1];
+  int64_t off = 0, end = g.off[1];
+#pragma unroll
+  for (int q = 1; q < 6; ++q) {
+    const bool in = t >= g.off[q];
+    off = in ? g.off[q] : off;
+    end = in ? g.off[q + 1] : end;
+    lx = in ? g.lo[q][0] : lx;
+    ly = in ? g.lo[q][1] : ly;
+    lz = in ? g.lo[q][2] : lz;
+    nx = in ? g.n[q][0] : nx;
+    ny = in ? g.n[q][1] : ny;
+  }
+  const int lo[3] = {lx, ly, lz};
+  box_cell(lo, nx, ny, end - off, t - off, iv);
 }
 
 // cell of the fab box at a linear index (x fastest)
 __device__ inline void fab_cell(const Fab& F, int64_t t, int iv[3]) {
-  const int nx = F.hi[0] - F.lo[0] + 1, ny = F.hi[1] - F.lo[1] + 1;
-  iv[0] = F.lo[0] + (int)(t % nx);
-  iv[1] = F.lo[1] + (int)((t / nx) % ny);
-  iv[2] = F.lo[2] + (int)(t / ((int64_t)nx * ny));
+  box_cell(F.lo, F.hi[0] - F.lo[0] + 1, F.hi[1] - F.lo[1] + 1, F.cells, t, iv);
+}
+
+// D's components at offset o = S's at offset p, eight loads in flight
+__device__ __forceinline__ void copy_comps(const Fab& S, int64_t p, const Fab& D, int64_t o, int nc) {
+  constexpr int kN = 8;
+  for (int n0 = 0; n0 < nc; n0 += kN) {
+    double v[kN];
+#pragma unroll
+    for (int u = 0; u < kN; ++u) v[u] = (n0 + u < nc) ? S.p[p + (int64_t)(n0 + u) * S.ns] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kN; ++u)
+      if (n0 + u < nc) D.p[o + (int64_t)(n0 + u) * D.ns] = v[u];
+  }
 }
 
 // InitEquilibrium (AmrCoreLBM.cpp:2146-2161) over a box
@@ -94,16 +178,16 @@ __global__ void k_box_equilibrium(Fab m, Fab f, int lo0, int lo1, int lo2, int n
 
 // FillBoundary of one box: ghost cells whose periodic image lies in the
 // valid box take its value (AMReX FillBoundary with the periodicity)
-__global__ void k_box_fill_periodic(Fab F, BoxGeom G) {
+__global__ void k_box_fill_periodic(Fab F, BoxGeom G, GhostBox gh) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= F.cells) return;
+  if (t >= gh.off[6]) return;
   int iv[3];
-  fab_cell(F, t, iv);
-  bool valid = true, perout = false;
+  ghost_cell(gh, t, iv);
+  bool perout = false;
   int s[3] = {iv[0], iv[1], iv[2]};
+#pragma unroll
   for (int d = 0; d < 3; ++d) {
     if (iv[d] >= G.vlo[d] && iv[d] <= G.vhi[d]) continue;
-    valid = false;
     if (d >= G.dim) return;
     const bool out = iv[d] < 0 || iv[d] > G.n[d] - 1;
     if (out && !G.periodic[d]) return;
@@ -114,75 +198,102 @@ __global__ void k_box_fill_periodic(Fab F, BoxGeom G) {
       s[d] = r;
     }
   }
-  if (valid || !perout) return;
+  if (!perout) return;
+#pragma unroll
   for (int d = 0; d < 3; ++d)
     if (s[d] < G.vlo[d] || s[d] > G.vhi[d]) return;
-  for (int n = 0; n < F.nc; ++n) F.at(iv[0], iv[1], iv[2], n) = F.at(s[0], s[1], s[2], n);
+  copy_comps(F, F.off(s[0], s[1], s[2]), F, F.off(iv[0], iv[1], iv[2]), F.nc);
 }
 
 // One pass of the physical BC fill (cells outside the domain in `pass`
 // non-periodic dimensions): FilccCell's foextrap copies (the last foextrap
 // dimension wins), then mesoscopicBcFill (meso) or macroBcFill.
 template <class LAT>
-__global__ void k_box_fill_physical(Fab F, BoxGeom G, int pass, int meso) {
+__device__ __forceinline__ void meso_ghost(int kind, const double* b, const double fnp[LAT::Q], double out[LAT::Q]);
+
+// the face whose functor sets a ghost cell: the first dimension, low side
+// first, of the given type that the cell is outside of; b: its boundary
+// values.  (Loops over the dimensions here and below are unrolled, so that
+// kernel arguments and cells are indexed by constants and stay in registers.)
+__device__ inline bool first_face(const BoxGeom& G, const int iv[3], int type, double b[4]) {
+  bool found = false;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= G.dim || found) continue;
+    const bool lo = iv[d] < 0 && G.lo_t[d] == type, hi = iv[d] > G.n[d] - 1 && G.hi_t[d] == type;
+    if (!lo && !hi) continue;
+    found = true;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[c] = lo ? G.lo_v[d][c] : G.hi_v[d][c];
+  }
+  return found;
+}
+
+template <class LAT>
+__global__ void k_box_fill_physical(Fab F, BoxGeom G, GhostBox gh, int pass, int meso) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= F.cells) return;
+  if (t >= gh.off[6]) return;
   int iv[3];
-  fab_cell(F, t, iv);
+  ghost_cell(gh, t, iv);
   if (nonper_out_cnt(G, iv) != pass) return;
   const int nc = F.nc;
-  for (int d = 0; d < G.dim; ++d) {
+  const int64_t o = F.off(iv[0], iv[1], iv[2]);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= G.dim) continue;
     int src[3] = {iv[0], iv[1], iv[2]};
     bool hit = false;
     if (iv[d] < 0 && G.lo_t[d] == BC_FOEXTRAP) { src[d] = 0; hit = true; }
     else if (iv[d] > G.n[d] - 1 && G.hi_t[d] == BC_FOEXTRAP) { src[d] = G.n[d] - 1; hit = true; }
-    if (hit)
-      for (int n = 0; n < nc; ++n) F.at(iv[0], iv[1], iv[2], n) = F.at(src[0], src[1], src[2], n);
+    if (hit) copy_comps(F, F.off(src[0], src[1], src[2]), F, o, nc);
   }
   // nearest interior cell, clamped in every dimension (bc_fill.H:15-41)
-  int mir[3] = {iv[0], iv[1], iv[2]}, lh[3] = {0, 0, 0}, hh[3] = {0, 0, 0};
-  for (int d = 0; d < G.dim; ++d) {
-    if (iv[d] < 0) { mir[d] = 0; lh[d] = 1; }
-    else if (iv[d] > G.n[d] - 1) { mir[d] = G.n[d] - 1; hh[d] = 1; }
+  int mir[3] = {iv[0], iv[1], iv[2]};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d >= G.dim) continue;
+    if (iv[d] < 0) mir[d] = 0;
+    else if (iv[d] > G.n[d] - 1) mir[d] = G.n[d] - 1;
   }
-  auto first_face = [&](int type, int* bd, int* lo_side) {
-    for (int d = 0; d < G.dim; ++d) {
-      if (lh[d] && G.lo_t[d] == type) { *bd = d; *lo_side = 1; return true; }
-      if (hh[d] && G.hi_t[d] == type) { *bd = d; *lo_side = 0; return true; }
-    }
-    return false;
-  };
-  int bd = -1, los = 1;
+  const int64_t m = F.off(mir[0], mir[1], mir[2]);
+  double b[4] = {0.0, 0.0, 0.0, 0.0};
   if (!meso) {  // macroBcFill (bc_fill.H:263-301)
-    if (first_face(BC_USER_2, &bd, &los)) {
-      const double* b = los ? G.lo_v[bd] : G.hi_v[bd];
-      for (int n = 0; n < nc; ++n) F.at(iv[0], iv[1], iv[2], n) = F.at(mir[0], mir[1], mir[2], n);
-      if (nc > 0) F.at(iv[0], iv[1], iv[2], 0) = fmax(1.0e-20, 2.0 * b[0] - F.at(mir[0], mir[1], mir[2], 0));
-      for (int n = 1; n < 4 && n < nc; ++n) F.at(iv[0], iv[1], iv[2], n) = 2.0 * b[n] - F.at(mir[0], mir[1], mir[2], n);
+    if (first_face(G, iv, BC_USER_2, b)) {
+      copy_comps(F, m, F, o, nc);
+      if (nc > 0) F.p[o] = fmax(1.0e-20, 2.0 * b[0] - F.p[m]);
+      for (int n = 1; n < 4 && n < nc; ++n) F.p[o + n * F.ns] = 2.0 * b[n] - F.p[m + n * F.ns];
       return;
     }
-    if (first_face(BC_USER_1, &bd, &los) || first_face(BC_EXT_DIR, &bd, &los)) {
-      const double* b = los ? G.lo_v[bd] : G.hi_v[bd];
-      for (int n = 0; n < nc; ++n) F.at(iv[0], iv[1], iv[2], n) = F.at(mir[0], mir[1], mir[2], n);
-      for (int n = 0; n < 4 && n < nc; ++n) F.at(iv[0], iv[1], iv[2], n) = b[n];
+    if (first_face(G, iv, BC_USER_1, b) || first_face(G, iv, BC_EXT_DIR, b)) {
+      copy_comps(F, m, F, o, nc);
+      for (int n = 0; n < 4 && n < nc; ++n) F.p[o + n * F.ns] = b[n];
     }
     return;
   }
   int kind = 0;
-  if (first_face(BC_USER_2, &bd, &los)) kind = 2;
-  else if (first_face(BC_USER_1, &bd, &los)) kind = 1;
-  else if (first_face(BC_EXT_DIR, &bd, &los)) kind = 3;
+  if (first_face(G, iv, BC_USER_2, b)) kind = BC_USER_2;
+  else if (first_face(G, iv, BC_USER_1, b)) kind = BC_USER_1;
+  else if (first_face(G, iv, BC_EXT_DIR, b)) kind = BC_EXT_DIR;
   if (kind == 0) return;
-  if (kind == 1) {  // copyMesoscopicFromMirror (:147-154)
-#pragma unroll
-    for (int q = 0; q < LAT::Q; ++q) F.at(iv[0], iv[1], iv[2], q) = F.at(mir[0], mir[1], mir[2], q);
+  if (kind == BC_USER_1) {  // copyMesoscopicFromMirror (:147-154)
+    copy_comps(F, m, F, o, LAT::Q);
     return;
   }
-  double fnp[LAT::Q];
+  double fnp[LAT::Q], out[LAT::Q];
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) fnp[q] = F.p[m + q * F.ns];
+  meso_ghost<LAT>(kind, b, fnp, out);
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) F.p[o + q * F.ns] = out[q];
+}
+
+// applyExtDirMesoscopic (:159-204) and applyFaceMirroredMesoscopic (:209-261)
+// from the populations fnp of the mirror cell
+template <class LAT>
+__device__ __forceinline__ void meso_ghost(int kind, const double* b, const double fnp[LAT::Q], double out[LAT::Q]) {
   double rhonp = 0.0, unp = 0.0, vnp = 0.0, wnp = 0.0;
 #pragma unroll
   for (int q = 0; q < LAT::Q; ++q) {
-    fnp[q] = F.at(mir[0], mir[1], mir[2], q);
     rhonp += fnp[q];
     unp += double(LAT::cx[q]) * fnp[q];
     vnp += double(LAT::cy[q]) * fnp[q];
@@ -190,14 +301,13 @@ __global__ void k_box_fill_physical(Fab F, BoxGeom G, int pass, int meso) {
   }
   rhonp = fmax(rhonp, 1.0e-20);
   unp /= rhonp; vnp /= rhonp; wnp /= rhonp;
-  const double* b = los ? G.lo_v[bd] : G.hi_v[bd];
   double rg = b[0], ug = b[1], vg = b[2], wg = b[3];
-  if (kind == 2) {  // applyFaceMirroredMesoscopic (:209-261)
+  if (kind == BC_USER_2) {
     rg = fmax(1.0e-20, 2.0 * b[0] - rhonp);
     ug = 2.0 * b[1] - unp; vg = 2.0 * b[2] - vnp; wg = 2.0 * b[3] - wnp;
   }
 #pragma unroll
-  for (int q = 0; q < LAT::Q; ++q) {  // applyExtDirMesoscopic (:159-204) / mirrored
+  for (int q = 0; q < LAT::Q; ++q) {
     const double cx = LAT::cx[q], cy = LAT::cy[q], cz = LAT::cz[q];
     const double eu_np = cx * unp + cy * vnp + cz * wnp;
     const double uv_np = unp * unp + vnp * vnp + wnp * wnp;
@@ -205,45 +315,233 @@ __global__ void k_box_fill_physical(Fab F, BoxGeom G, int pass, int meso) {
     const double eu_g = cx * ug + cy * vg + cz * wg;
     const double uv_g = ug * ug + vg * vg + wg * wg;
     const double feqg = LAT::w[q] * rg * (1.0 + 3.0 * eu_g + 4.5 * eu_g * eu_g - 1.5 * uv_g);
-    F.at(iv[0], iv[1], iv[2], q) = feqg + (fnp[q] - feqnp);
+    out[q] = feqg + (fnp[q] - feqnp);
   }
+}
+
+// Where FillPatch of a level of one box takes a ghost cell from, once every
+// pass above has run on a fab that was zero outside its valid cells.  false:
+// the cell stays zero; true: src, with kind 0 a copy, else the functor of
+// boundary values b applied to it (sv false: src is not valid, to zeros).
+// per: a periodic image of a valid cell.
+struct PatchSource {
+  int src[3], kind;
+  double b[4];
+  bool sv, per;
+};
+__device__ inline bool patch_source(const BoxGeom& G, const int iv[3], PatchSource& P) {
+  bool out = false, nonper = false;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    P.src[d] = iv[d];
+    if (d < G.dim && (iv[d] < 0 || iv[d] > G.n[d] - 1)) {
+      out = true;
+      if (!G.periodic[d]) nonper = true;
+    }
+  }
+  P.kind = 0;
+  P.sv = true;
+  P.per = out && !nonper;
+  if (!out) return false;
+  if (nonper) {
+    if (first_face(G, iv, BC_USER_2, P.b)) P.kind = BC_USER_2;
+    else if (first_face(G, iv, BC_USER_1, P.b)) P.kind = BC_USER_1;
+    else if (first_face(G, iv, BC_EXT_DIR, P.b)) P.kind = BC_EXT_DIR;
+    // the mirror clamps every dimension; foextrap the non-periodic ones, if
+    // the cell is outside of no other kind of face
+    bool other = false;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if (d >= G.dim || (P.kind == 0 && G.periodic[d])) continue;
+      if (iv[d] < 0) { P.src[d] = 0; other = other || G.lo_t[d] != BC_FOEXTRAP; }
+      else if (iv[d] > G.n[d] - 1) { P.src[d] = G.n[d] - 1; other = other || G.hi_t[d] != BC_FOEXTRAP; }
+    }
+    if (P.kind == 0 && other) return false;
+  }
+  bool valid = true;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    if (d < G.dim && P.kind == 0 && G.periodic[d] && (P.src[d] < 0 || P.src[d] > G.n[d] - 1)) {
+      P.src[d] %= G.n[d];
+      if (P.src[d] < 0) P.src[d] += G.n[d];
+    }
+    valid = valid && P.src[d] >= G.vlo[d] && P.src[d] <= G.vhi[d];
+  }
+  P.sv = valid;
+  return valid || P.kind != 0;
+}
+
+// The cells of a pass over a level of one box, x fastest: those of the fab or
+// of its valid box.  A pass that writes ghost cells runs over whole fab rows:
+// a row's last valid cells share a cache line with its ghosts and the next
+// row's, and a line written in parts by different blocks costs more than
+// the few lanes of a wavefront that take the ghost path beside valid ones
+// (fill_collide 128x96x96: 138 us with valid and ghost cells in blocks of
+// their own, 114 in rows).
+struct PassBox {
+  int lo[3], nx, ny;
+  int64_t cells;
+};
+static PassBox pass_box(const int lo[3], const int hi[3]) {
+  PassBox p{};
+  for (int d = 0; d < 3; ++d) p.lo[d] = lo[d];
+  p.nx = hi[0] - lo[0] + 1;
+  p.ny = hi[1] - lo[1] + 1;
+  p.cells = (int64_t)p.nx * p.ny * (hi[2] - lo[2] + 1);
+  return p;
+}
+__device__ inline bool pass_cell(const PassBox& pb, const BoxGeom& G, bool* ghost, int iv[3]) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= pb.cells) return false;
+  box_cell(pb.lo, pb.nx, pb.ny, pb.cells, t, iv);
+  *ghost = false;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) *ghost = *ghost || iv[d] < G.vlo[d] || iv[d] > G.vhi[d];
+  return true;
+}
+
+// FillPatchSingleLevel of a level of one box in one pass over the fab: the
+// valid cells of S, their periodic images, the physical ghost values and
+// zeros elsewhere, in place of a fill with zeros, a copy, a periodic and up
+// to three physical passes.
+template <class LAT>
+__global__ void __launch_bounds__(256) k_box_fill_patch(Fab S, Fab D, BoxGeom G, PassBox pb, int meso) {
+  int iv[3];
+  bool ghost;
+  if (!pass_cell(pb, G, &ghost, iv)) return;
+  const int64_t o = D.off(iv[0], iv[1], iv[2]);
+  const int nc = D.nc;
+  if (!ghost) {
+    copy_comps(S, S.off(iv[0], iv[1], iv[2]), D, o, nc);
+    return;
+  }
+  PatchSource P;
+  const bool any = patch_source(G, iv, P);
+  const int64_t p = P.sv ? S.off(P.src[0], P.src[1], P.src[2]) : 0;
+  if (!any || (!P.sv && meso && P.kind == BC_USER_1)) {
+    for (int n = 0; n < nc; ++n) D.p[o + n * D.ns] = 0.0;
+    return;
+  }
+  if (P.kind == 0 || (meso && P.kind == BC_USER_1)) {
+    copy_comps(S, p, D, o, nc);
+    return;
+  }
+  if (!meso) {  // macroBcFill
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      if (n >= nc) continue;
+      const double m = P.sv ? S.p[p + n * S.ns] : 0.0;
+      const double r = 2.0 * P.b[n] - m;
+      D.p[o + n * D.ns] = (P.kind != BC_USER_2) ? P.b[n] : (n == 0) ? fmax(1.0e-20, r) : r;
+    }
+    for (int n = 4; n < nc; ++n) D.p[o + n * D.ns] = P.sv ? S.p[p + n * S.ns] : 0.0;
+    return;
+  }
+  double fnp[LAT::Q], out[LAT::Q];
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) fnp[q] = P.sv ? S.p[p + q * S.ns] : 0.0;
+  meso_ghost<LAT>(P.kind, P.b, fnp, out);
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) D.p[o + q * D.ns] = out[q];
+  for (int n = LAT::Q; n < nc; ++n) D.p[o + n * D.ns] = P.sv ? S.p[p + n * S.ns] : 0.0;
+}
+
+template <class LAT>
+static void launch_fill_patch(const Fab& S, const Fab& D, const BoxGeom& G, int meso, hipStream_t s) {
+  const PassBox pb = pass_box(D.lo, D.hi);
+  hipLaunchKernelGGL(k_box_fill_patch<LAT>, dim3((unsigned)((pb.cells + 255) / 256)), dim3(256), 0, s, S, D, G, pb,
+                     meso);
 }
 
 // collide / collide_forced over the valid box (AdvanceLBMAtLevel.cpp:196-240)
 template <class LAT>
-__global__ void k_box_collide(Fab f, Fab m, Fab F, double tau, BoxGeom G) {
-  const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
-  const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= cells) return;
-  const int i = G.vlo[0] + (int)(t % nx), j = G.vlo[1] + (int)((t / nx) % ny);
-  const int k = G.vlo[2] + (int)(t / ((int64_t)nx * ny));
-  const double rho = m.at(i, j, k, 0), u = m.at(i, j, k, 1), v = m.at(i, j, k, 2), w = m.at(i, j, k, 3);
-  const double fx = F.p ? F.at(i, j, k, 0) : 0.0, fy = F.p ? F.at(i, j, k, 1) : 0.0;
-  const double fz = F.p ? F.at(i, j, k, 2) : 0.0;
+__device__ __forceinline__ void collide_cell(const Fab& S, const Fab& m, const Fab& F, double tau, int i, int j, int k,
+                                             double g[LAT::Q]) {
+  const int64_t p = S.off(i, j, k), pm = m.off(i, j, k);
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) g[q] = S.p[p + q * S.ns];
+  const double rho = m.p[pm], u = m.p[pm + m.ns], v = m.p[pm + 2 * m.ns], w = m.p[pm + 3 * m.ns];
+  double fx = 0.0, fy = 0.0, fz = 0.0;
+  if (F.p) {
+    const int64_t pf = F.off(i, j, k);
+    fx = F.p[pf];
+    fy = F.p[pf + F.ns];
+    fz = F.p[pf + 2 * F.ns];
+  }
   const double uv = usq<LAT, double>(u, v, w);
   const bool forced = !(fx == 0.0 && fy == 0.0 && fz == 0.0);
   const double fac = 1.0 - 0.5 / tau;
 #pragma unroll
   for (int q = 0; q < LAT::Q; ++q) {
     const double fe = feq_q<LAT, double>(q, rho, u, v, w, uv);
-    double g = bgk<StF64>(f.at(i, j, k, q), fe, tau, 1.0 / tau);
-    if (forced) g += guo_q<LAT, double>(q, fac, u, v, w, fx, fy, fz);
-    f.at(i, j, k, q) = g;
+    g[q] = bgk<StF64>(g[q], fe, tau, 1.0 / tau);
+    if (forced) g[q] += guo_q<LAT, double>(q, fac, u, v, w, fx, fy, fz);
   }
+}
+
+template <class LAT>
+__global__ void __launch_bounds__(256) k_box_collide(Fab f, Fab m, Fab F, double tau, BoxGeom G) {
+  const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
+  const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= cells) return;
+  int iv[3];
+  box_cell(G.vlo, nx, ny, cells, t, iv);
+  double g[LAT::Q];
+  collide_cell<LAT>(f, m, F, tau, iv[0], iv[1], iv[2], g);
+  const int64_t o = f.off(iv[0], iv[1], iv[2]);
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) f.p[o + q * f.ns] = g[q];
+}
+
+// FillPatch, collide and FillBoundary of a level of one box in one pass: D's
+// valid cells are S's collided, its periodic ghosts their images (collided
+// again by the ghost's own thread), its other ghosts FillPatch's values of S
+// (pre-collision); only the valid cells where pb is their box.  Reads S and
+// writes D once, where the separate stages wrote the fab with zeros, copied,
+// filled and collided it in place (128x96x96 D3Q19: 114 us; zeros 64, copy 88,
+// fills 60, collision 75 before).  Bound by HBM: the sweep's 460 MB at 4 TB/s.
+template <class LAT>
+__global__ void __launch_bounds__(256) k_box_fill_collide(Fab S, Fab D, Fab m, Fab F, double tau, BoxGeom G,
+                                                          PassBox pb) {
+  int iv[3];
+  bool ghost;
+  if (!pass_cell(pb, G, &ghost, iv)) return;
+  const int64_t o = D.off(iv[0], iv[1], iv[2]);
+  double g[LAT::Q];
+  PatchSource P;
+  bool collide = true;
+  if (ghost) {
+    const bool any = patch_source(G, iv, P);
+    collide = any && P.per;
+    if (!collide) {
+      double fnp[LAT::Q];
+      const int64_t p = (any && P.sv) ? S.off(P.src[0], P.src[1], P.src[2]) : 0;
+#pragma unroll
+      for (int q = 0; q < LAT::Q; ++q) fnp[q] = (any && P.sv) ? S.p[p + q * S.ns] : 0.0;
+      if (any && (P.kind == BC_USER_2 || P.kind == BC_EXT_DIR)) {
+        meso_ghost<LAT>(P.kind, P.b, fnp, g);
+      } else {
+#pragma unroll
+        for (int q = 0; q < LAT::Q; ++q) g[q] = fnp[q];
+      }
+    } else {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) iv[d] = P.src[d];
+    }
+  }
+  if (collide) collide_cell<LAT>(S, m, F, tau, iv[0], iv[1], iv[2], g);
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) D.p[o + q * D.ns] = g[q];
 }
 
 // halfway bounce-back into user_1 ghost cells (AdvanceLBMAtLevel.cpp:265-373)
 template <class LAT>
-__global__ void k_box_bounce_back(Fab f, BoxGeom G) {
+__global__ void k_box_bounce_back(Fab f, BoxGeom G, GhostBox gh) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= f.cells) return;
+  if (t >= gh.off[6]) return;
   int iv[3];
-  fab_cell(f, t, iv);
-  bool valid = true;
-  for (int d = 0; d < 3; ++d)
-    if (iv[d] < G.vlo[d] || iv[d] > G.vhi[d]) valid = false;
-  if (valid) return;
+  ghost_cell(gh, t, iv);
   bool has_bb = false, unsup = false;
   for (int d = 0; d < G.dim; ++d) {
     if (iv[d] < 0) { if (G.lo_t[d] == BC_USER_1) has_bb = true; else unsup = true; }
@@ -261,29 +559,38 @@ __global__ void k_box_bounce_back(Fab f, BoxGeom G) {
 // stream (stream.H:9-22) and calculateMacroForcing
 // (calculateMacroForcing.H:9-32) over the valid box
 template <class LAT>
-__global__ void k_box_stream_macro(Fab fin, Fab fout, Fab mout, Fab F, BoxGeom G) {
+__global__ void __launch_bounds__(256) k_box_stream_macro(Fab fin, Fab fout, Fab mout, Fab F, BoxGeom G) {
   const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
   const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cells) return;
-  const int i = G.vlo[0] + (int)(t % nx), j = G.vlo[1] + (int)((t / nx) % ny);
-  const int k = G.vlo[2] + (int)(t / ((int64_t)nx * ny));
+  int iv[3];
+  box_cell(G.vlo, nx, ny, cells, t, iv);
+  const int64_t p = fin.off(iv[0], iv[1], iv[2]), o = fout.off(iv[0], iv[1], iv[2]), om = mout.off(iv[0], iv[1], iv[2]);
+  double f[LAT::Q];
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) f[q] = fin.p[p - LAT::cx[q] - LAT::cy[q] * fin.js - LAT::cz[q] * fin.ks + q * fin.ns];
+  double fx = 0.0, fy = 0.0, fz = 0.0;
+  if (F.p) {
+    const int64_t pf = F.off(iv[0], iv[1], iv[2]);
+    fx = F.p[pf];
+    fy = F.p[pf + F.ns];
+    fz = F.p[pf + 2 * F.ns];
+  }
   double r = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
 #pragma unroll
   for (int q = 0; q < LAT::Q; ++q) {
-    const double fq = fin.at(i - LAT::cx[q], j - LAT::cy[q], k - LAT::cz[q], q);
-    fout.at(i, j, k, q) = fq;
-    r += fq;
-    m1 += double(LAT::cx[q]) * fq;
-    m2 += double(LAT::cy[q]) * fq;
-    m3 += double(LAT::cz[q]) * fq;
+    r += f[q];
+    m1 += double(LAT::cx[q]) * f[q];
+    m2 += double(LAT::cy[q]) * f[q];
+    m3 += double(LAT::cz[q]) * f[q];
   }
-  const double fx = F.p ? F.at(i, j, k, 0) : 0.0, fy = F.p ? F.at(i, j, k, 1) : 0.0;
-  const double fz = F.p ? F.at(i, j, k, 2) : 0.0;
-  mout.at(i, j, k, 0) = r;
-  mout.at(i, j, k, 1) = (m1 + 0.5 * fx) / r;
-  mout.at(i, j, k, 2) = (m2 + 0.5 * fy) / r;
-  mout.at(i, j, k, 3) = (m3 + 0.5 * fz) / r;
+#pragma unroll
+  for (int q = 0; q < LAT::Q; ++q) fout.p[o + q * fout.ns] = f[q];
+  mout.p[om] = r;
+  mout.p[om + mout.ns] = (m1 + 0.5 * fx) / r;
+  mout.p[om + 2 * mout.ns] = (m2 + 0.5 * fy) / r;
+  mout.p[om + 3 * mout.ns] = (m3 + 0.5 * fz) / r;
 }
 
 // vorticity and pressure (visPara.H:10-54) from a macro patch with one ghost
@@ -292,8 +599,9 @@ __global__ void k_box_derived(Fab mp, Fab mout, BoxGeom G, double dx, double dy,
   const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cells) return;
-  const int i = G.vlo[0] + (int)(t % nx), j = G.vlo[1] + (int)((t / nx) % ny);
-  const int k = G.vlo[2] + (int)(t / ((int64_t)nx * ny));
+  int iv[3];
+  box_cell(G.vlo, nx, ny, cells, t, iv);
+  const int i = iv[0], j = iv[1], k = iv[2];
   const double P = (mp.at(i, j, k, 0) - 1.0) / 3.0;
   const double dv_dx = (mp.at(i + 1, j, k, 2) - mp.at(i - 1, j, k, 2)) / (2.0 * dx);
   const double du_dy = (mp.at(i, j + 1, k, 1) - mp.at(i, j - 1, k, 1)) / (2.0 * dy);
@@ -313,6 +621,7 @@ __global__ void k_box_derived(Fab mp, Fab mout, BoxGeom G, double dx, double dy,
 }
 
 // per-block partial sums of one component over a box, fixed order
+// (blockIdx.y: component comp + blockIdx.y, its partials gridDim.x + 1 apart)
 __global__ void __launch_bounds__(256) k_box_sum(Fab F, int comp, BoxGeom G, double* partial) {
   __shared__ double lds[4];
   const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
@@ -320,14 +629,23 @@ __global__ void __launch_bounds__(256) k_box_sum(Fab F, int comp, BoxGeom G, dou
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   double v = 0.0;
   if (t < cells) {
-    const int i = G.vlo[0] + (int)(t % nx), j = G.vlo[1] + (int)((t / nx) % ny);
-    const int k = G.vlo[2] + (int)(t / ((int64_t)nx * ny));
-    v = F.at(i, j, k, comp);
+    int iv[3];
+    box_cell(G.vlo, nx, ny, cells, t, iv);
+    v = F.at(iv[0], iv[1], iv[2], comp + (int)blockIdx.y);
   }
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) partial[blockIdx.x] = ((lds[0] + lds[1]) + lds[2]) + lds[3];
+  if (threadIdx.x == 0)
+    partial[(int64_t)blockIdx.y * (gridDim.x + 1) + blockIdx.x] = ((lds[0] + lds[1]) + lds[2]) + lds[3];
+}
+
+// the sums of k_box_sum's partials behind each component's: block c adds the
+// nb partials of component c (k_sum_partials)
+__global__ void __launch_bounds__(1024) k_box_sum_partials(double* partial, int64_t nb) {
+  double* p = partial + (int64_t)blockIdx.x * (nb + 1);
+  const double r = sum_partials_body(p, nb);
+  if (threadIdx.x == 0) p[nb] = r;
 }
 
 static BoxGeom box_geom(const ilbm_case_desc& c, const int* vlo, const int* vhi) {
@@ -376,6 +694,18 @@ static void check_fab(const ilbm_fab* f, int min_comp, const BoxGeom& G, int gho
   }
 }
 
+// a dense array [nc][cells] of a domain without ghost cells
+static Fab cells_fab(double* p, const ilbm_case_desc& c, int nc) {
+  Fab F{};
+  F.p = p;
+  for (int d = 0; d < 3; ++d) F.hi[d] = (d < c.dim) ? c.n[d] - 1 : 0;
+  F.js = c.n[0];
+  F.ks = (int64_t)c.n[0] * c.n[1];
+  F.ns = F.cells = F.ks * (F.hi[2] + 1);
+  F.nc = nc;
+  return F;
+}
+
 // macro (rho, ux, uy, uz; [4][cells], no ghosts) into the interior of a fab
 __global__ void k_fab_from_cells(Fab F, const double* m, int nx, int ny, int64_t cells) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -391,23 +721,40 @@ __global__ void k_cells_from_fab(Fab F, int comp0, int ncomp, double* out, int n
   for (int n = 0; n < ncomp; ++n) out[n * cells + t] = F.at(i, j, k, comp0 + n);
 }
 
+// the physical fill's passes: one per non-periodic dimension the fab leaves
+template <class LAT>
+static void launch_fill_physical(const Fab& F, const BoxGeom& G, int meso, hipStream_t s) {
+  int dlo[3] = {0, 0, 0}, dhi[3], passes = 0;
+  for (int d = 0; d < 3; ++d) {
+    dhi[d] = G.n[d] - 1;
+    if (d >= G.dim) { dlo[d] = F.lo[d]; dhi[d] = F.hi[d]; }
+    else if (!G.periodic[d] && (F.lo[d] < 0 || F.hi[d] > G.n[d] - 1)) ++passes;
+  }
+  if (passes == 0) return;
+  const GhostBox gh = ghost_box(F, dlo, dhi);
+  if (gh.off[6] == 0) return;
+  for (int pass = 1; pass <= passes; ++pass)
+    hipLaunchKernelGGL(k_box_fill_physical<LAT>, grid_for(gh.off[6]), dim3(256), 0, s, F, G, gh, pass, meso);
+}
+
 // ParallelCopy of a box region between two fabs (same index space)
 __global__ void k_box_copy(Fab S, Fab D, BoxGeom G, int ncomp) {
   const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
   const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= cells) return;
-  const int i = G.vlo[0] + (int)(t % nx), j = G.vlo[1] + (int)((t / nx) % ny);
-  const int k = G.vlo[2] + (int)(t / ((int64_t)nx * ny));
-  for (int n = 0; n < ncomp; ++n) D.at(i, j, k, n) = S.at(i, j, k, n);
+  int iv[3];
+  box_cell(G.vlo, nx, ny, cells, t, iv);
+  const int i = iv[0], j = iv[1], k = iv[2];
+  copy_comps(S, S.off(i, j, k), D, D.off(i, j, k), ncomp);
 }
 
 __global__ void k_fab_setval(Fab F, double v) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= F.cells * F.nc) return;
+  if (t >= F.cells) return;
   int iv[3];
-  fab_cell(F, t % F.cells, iv);
-  F.at(iv[0], iv[1], iv[2], (int)(t / F.cells)) = v;
+  fab_cell(F, t, iv);
+  F.at(iv[0], iv[1], iv[2], (int)blockIdx.y) = v;
 }
 
 }  // namespace ilbm
@@ -438,7 +785,7 @@ int ilbm_box_setval(ilbm_fab* f, double value, void* stream) {
   return guarded([&] {
     using namespace ilbm;
     const Fab F = to_fab(*f);
-    hipLaunchKernelGGL(k_fab_setval, grid_for(F.cells * F.nc), dim3(256), 0, (hipStream_t)stream, F, value);
+    hipLaunchKernelGGL(k_fab_setval, dim3(grid_for(F.cells).x, (unsigned)F.nc), dim3(256), 0, (hipStream_t)stream, F, value);
     HIPCHK(hipGetLastError());
   });
 }
@@ -496,13 +843,10 @@ int ilbm_level_get_derived(ilbm_level* h, double* host_out) {
     const BoxGeom G = box_geom(c, nullptr, nullptr);
     const int64_t cells = L.ncells;
     hipStream_t s = L.stream;
-    hipLaunchKernelGGL(k_fab_from_cells, grid_for(cells), dim3(256), 0, s, P, (const double*)L.mout, c.n[0], c.n[1],
-                       cells);
-    hipLaunchKernelGGL(k_box_fill_periodic, grid_for(P.cells), dim3(256), 0, s, P, G);
+    const Fab S = cells_fab(L.mout, c, 4);
     with_lattice(L.lat, [&](auto lat) {
       using LAT = decltype(lat);
-      for (int pass = 1; pass <= c.dim; ++pass)
-        hipLaunchKernelGGL(k_box_fill_physical<LAT>, grid_for(P.cells), dim3(256), 0, s, P, G, pass, 0);
+      launch_fill_patch<LAT>(S, P, G, 0, s);
     });
     hipLaunchKernelGGL(k_box_derived, grid_for(cells), dim3(256), 0, s, P, O, G, c.dx[0], c.dx[1], c.dx[2]);
     double* outd = dev_alloc<double>(2 * cells);
@@ -542,7 +886,14 @@ int ilbm_box_fill_periodic(const ilbm_case_desc* d, ilbm_fab* fab, const int vlo
     using namespace ilbm;
     const BoxGeom G = box_geom(*d, vlo, vhi);
     const Fab F = to_fab(*fab);
-    hipLaunchKernelGGL(k_box_fill_periodic, grid_for(F.cells), dim3(256), 0, (hipStream_t)stream, F, G);
+    // only cells outside the domain in a periodic dimension are filled
+    bool any = false;
+    for (int e = 0; e < d->dim; ++e)
+      if (G.periodic[e] && (F.lo[e] < 0 || F.hi[e] > G.n[e] - 1)) any = true;
+    if (!any) return;
+    const GhostBox gh = ghost_box(F, G.vlo, G.vhi);
+    if (gh.off[6] == 0) return;
+    hipLaunchKernelGGL(k_box_fill_periodic, grid_for(gh.off[6]), dim3(256), 0, (hipStream_t)stream, F, G, gh);
     HIPCHK(hipGetLastError());
   });
 }
@@ -556,9 +907,7 @@ int ilbm_box_fill_physical(const ilbm_case_desc* d, ilbm_fab* fab, int mesoscopi
     if (mesoscopic && F.nc < d->q) throw StatusError{ILBM_ERR_INVALID, "mesoscopic fab needs q components"};
     with_lattice(box_lattice(*d), [&](auto L) {
       using LAT = decltype(L);
-      for (int pass = 1; pass <= d->dim; ++pass)
-        hipLaunchKernelGGL(k_box_fill_physical<LAT>, grid_for(F.cells), dim3(256), 0, (hipStream_t)stream, F, G,
-                           pass, mesoscopic ? 1 : 0);
+      launch_fill_physical<LAT>(F, G, mesoscopic ? 1 : 0, (hipStream_t)stream);
     });
     HIPCHK(hipGetLastError());
   });
@@ -584,6 +933,48 @@ int ilbm_box_collide(const ilbm_case_desc* d, ilbm_fab* f, const ilbm_fab* macro
   });
 }
 
+int ilbm_box_fill_patch(const ilbm_case_desc* d, const ilbm_fab* src, ilbm_fab* dst, int mesoscopic,
+                        const int vlo[3], const int vhi[3], void* stream) {
+  if (!d || !src || !dst || !vlo || !vhi) return ILBM_ERR_INVALID;
+  return guarded([&] {
+    using namespace ilbm;
+    const BoxGeom G = box_geom(*d, vlo, vhi);
+    check_fab(dst, mesoscopic ? d->q : 1, G, 0);
+    check_fab(src, dst->ncomp, G, 0);
+    if (src->p == dst->p) throw StatusError{ILBM_ERR_INVALID, "source and destination are one fab"};
+    const Fab S = to_fab(*src), D = to_fab(*dst);
+    with_lattice(box_lattice(*d), [&](auto L) {
+      using LAT = decltype(L);
+      launch_fill_patch<LAT>(S, D, G, mesoscopic ? 1 : 0, (hipStream_t)stream);
+    });
+    HIPCHK(hipGetLastError());
+  });
+}
+
+int ilbm_box_fill_collide(const ilbm_case_desc* d, const ilbm_fab* src, ilbm_fab* dst, const ilbm_fab* macro,
+                          const ilbm_fab* force, int ghosts, const int vlo[3], const int vhi[3], void* stream) {
+  if (!d || !src || !dst || !vlo || !vhi) return ILBM_ERR_INVALID;
+  return guarded([&] {
+    using namespace ilbm;
+    const BoxGeom G = box_geom(*d, vlo, vhi);
+    check_fab(src, d->q, G, 0);
+    check_fab(dst, d->q, G, 0);
+    check_fab(macro, 4, G, 0);
+    if (src->p == dst->p) throw StatusError{ILBM_ERR_INVALID, "source and destination are one fab"};
+    Fab Fo{};
+    if (force) { check_fab(force, 3, G, 0); Fo = to_fab(*force); }
+    const double tau = 3.0 * d->nu / d->dx[0] + 0.5;  // AmrCoreLBM.cpp:225-238
+    const Fab S = to_fab(*src), D = to_fab(*dst), M = to_fab(*macro);
+    const PassBox pb = ghosts ? pass_box(D.lo, D.hi) : pass_box(G.vlo, G.vhi);
+    with_lattice(box_lattice(*d), [&](auto L) {
+      using LAT = decltype(L);
+      hipLaunchKernelGGL(k_box_fill_collide<LAT>, grid_for(pb.cells), dim3(256), 0, (hipStream_t)stream, S, D, M, Fo,
+                         tau, G, pb);
+    });
+    HIPCHK(hipGetLastError());
+  });
+}
+
 int ilbm_box_bounce_back(const ilbm_case_desc* d, ilbm_fab* f, const int vlo[3], const int vhi[3], void* stream) {
   if (!d || !vlo || !vhi) return ILBM_ERR_INVALID;
   return guarded([&] {
@@ -591,9 +982,15 @@ int ilbm_box_bounce_back(const ilbm_case_desc* d, ilbm_fab* f, const int vlo[3],
     const BoxGeom G = box_geom(*d, vlo, vhi);
     check_fab(f, d->q, G, 1);
     const Fab F = to_fab(*f);
-    with_lattice(box_lattice(*d), [&](auto L) {
+    bool walls = false;   // only ghost cells beyond user_1 faces change
+    for (int e = 0; e < d->dim; ++e)
+      if (G.lo_t[e] == BC_USER_1 || G.hi_t[e] == BC_USER_1) walls = true;
+    const int lat = box_lattice(*d);
+    const GhostBox gh = ghost_box(F, G.vlo, G.vhi);
+    if (!walls || gh.off[6] == 0) return;
+    with_lattice(lat, [&](auto L) {
       using LAT = decltype(L);
-      hipLaunchKernelGGL(k_box_bounce_back<LAT>, grid_for(F.cells), dim3(256), 0, (hipStream_t)stream, F, G);
+      hipLaunchKernelGGL(k_box_bounce_back<LAT>, grid_for(gh.off[6]), dim3(256), 0, (hipStream_t)stream, F, G, gh);
     });
     HIPCHK(hipGetLastError());
   });
@@ -630,6 +1027,43 @@ int ilbm_box_derived(const ilbm_case_desc* d, const ilbm_fab* macro_patch, ilbm_
     hipLaunchKernelGGL(k_box_derived, grid_for(box_cells(G)), dim3(256), 0, (hipStream_t)stream,
                        to_fab(*macro_patch), to_fab(*macro_out), G, d->dx[0], d->dx[1], d->dx[2]);
     HIPCHK(hipGetLastError());
+  });
+}
+
+int ilbm_box_sums_workspace(const int vlo[3], const int vhi[3], int ncomp, int64_t* bytes) {
+  if (!vlo || !vhi || !bytes || ncomp < 1) return ILBM_ERR_INVALID;
+  int64_t cells = 1;
+  for (int e = 0; e < 3; ++e) {
+    if (vhi[e] < vlo[e]) return ILBM_ERR_INVALID;
+    cells *= vhi[e] - vlo[e] + 1;
+  }
+  *bytes = 8 * ncomp * ((cells + 255) / 256 + 1);
+  return ILBM_OK;
+}
+
+int ilbm_box_sums(const ilbm_fab* fab, int comp, int ncomp, const int vlo[3], const int vhi[3], void* work,
+                  int64_t work_bytes, double* host_out, void* stream) {
+  int64_t need = 0;
+  if (!fab || !fab->p || !work || !host_out || comp < 0 || ncomp < 1 || ncomp > 64 || comp + ncomp > fab->ncomp ||
+      ilbm_box_sums_workspace(vlo, vhi, ncomp, &need) != ILBM_OK || work_bytes < need)
+    return ILBM_ERR_INVALID;
+  return guarded([&] {
+    using namespace ilbm;
+    BoxGeom G{};
+    G.dim = 3;
+    for (int e = 0; e < 3; ++e) { G.vlo[e] = vlo[e]; G.vhi[e] = vhi[e]; }
+    const Fab F = to_fab(*fab);
+    if (!F.contains(vlo[0], vlo[1], vlo[2]) || !F.contains(vhi[0], vhi[1], vhi[2]))
+      throw StatusError{ILBM_ERR_INVALID, "box outside the fab"};
+    const int64_t nb = (box_cells(G) + 255) / 256;
+    double* part = static_cast<double*>(work);
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(k_box_sum, dim3((unsigned)nb, (unsigned)ncomp), dim3(256), 0, s, F, comp, G, part);
+    hipLaunchKernelGGL(k_box_sum_partials, dim3((unsigned)ncomp), dim3(1024), 0, s, part, nb);
+    HIPCHK(hipGetLastError());
+    // one strided copy of the sums behind each component's partials
+    HIPCHK(hipMemcpy2DAsync(host_out, 8, part + nb, 8 * (size_t)(nb + 1), 8, (size_t)ncomp, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
   });
 }
 
@@ -755,19 +1189,11 @@ __device__ inline void box_cf_cell(const Fab& Co, const Fab& Cn, const TimeMix& 
   }
 }
 
-// Interpolated macros on the cells of `dom` (the f fab's box when f is
-// given, else the macro fab's) inside (ghosts = 0) or outside (ghosts = 1)
-// the valid box; f = feq of them where f is given (ncomp >= 4 then).
+// Interpolated macros of one cell; f = feq of them where f is given
+// (ncomp >= 4 then).
 template <class LAT>
-__global__ void k_box_cf_fill(Fab Co, Fab Cn, TimeMix tm, Fab M, Fab Fq, Fab dom, int ncomp, BoxGeom G, int ghosts) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= dom.cells) return;
-  int iv[3];
-  fab_cell(dom, t, iv);
-  bool in_valid = true;
-  for (int d = 0; d < LAT::D; ++d)
-    if (iv[d] < G.vlo[d] || iv[d] > G.vhi[d]) in_valid = false;
-  if (in_valid == (ghosts != 0)) return;
+__device__ __forceinline__ void box_cf_comps(const Fab& Co, const Fab& Cn, const TimeMix& tm, const Fab& M,
+                                             const Fab& Fq, int ncomp, const int iv[3]) {
   switch (ncomp) {
     case 1: box_cf_cell<LAT, 1>(Co, Cn, tm, M, Fq, iv); break;
     case 2: box_cf_cell<LAT, 2>(Co, Cn, tm, M, Fq, iv); break;
@@ -780,6 +1206,39 @@ __global__ void k_box_cf_fill(Fab Co, Fab Cn, TimeMix tm, Fab M, Fab Fq, Fab dom
   }
 }
 
+// the ghost cells of a fine fab, a thread each; the blocks after nghost copy
+// the macros of the valid cells from Ms (where given)
+template <class LAT>
+__global__ void __launch_bounds__(256) k_box_cf_ghosts(Fab Co, Fab Cn, TimeMix tm, Fab M, Fab Fq, Fab Ms, int ncomp,
+                                                       BoxGeom G, GhostBox gh, unsigned nghost) {
+  int iv[3];
+  if (blockIdx.x >= nghost) {
+    const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
+    const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
+    const int64_t t = (int64_t)(blockIdx.x - nghost) * blockDim.x + threadIdx.x;
+    if (t >= cells) return;
+    box_cell(G.vlo, nx, ny, cells, t, iv);
+    copy_comps(Ms, Ms.off(iv[0], iv[1], iv[2]), M, M.off(iv[0], iv[1], iv[2]), ncomp);
+    return;
+  }
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= gh.off[6]) return;
+  ghost_cell(gh, t, iv);
+  box_cf_comps<LAT>(Co, Cn, tm, M, Fq, ncomp, iv);
+}
+
+// every cell of the valid box
+template <class LAT>
+__global__ void __launch_bounds__(256) k_box_cf_valid(Fab C, Fab M, int ncomp, BoxGeom G) {
+  const int nx = G.vhi[0] - G.vlo[0] + 1, ny = G.vhi[1] - G.vlo[1] + 1;
+  const int64_t cells = (int64_t)nx * ny * (G.vhi[2] - G.vlo[2] + 1);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= cells) return;
+  int iv[3];
+  box_cell(G.vlo, nx, ny, cells, t, iv);
+  box_cf_comps<LAT>(C, C, TimeMix{1, 0.0, 0.0}, M, Fab{}, ncomp, iv);
+}
+
 // amrex::average_down of f (Q comps) and macros (nmac comps) over the coarse
 // cells [clo, clo + cn): crse = (sum of the children, k then j then i) / 2^d
 template <class LAT>
@@ -787,24 +1246,26 @@ __global__ void k_box_average_down(Fab Ff, Fab Mf, Fab Fc, Fab Mc, int nmac, int
                                    int cny, int64_t ncov) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= ncov) return;
-  const int i = clo0 + (int)(t % cnx), j = clo1 + (int)((t / cnx) % cny), k = clo2 + (int)(t / ((int64_t)cnx * cny));
+  int civ[3];
+  const int clo[3] = {clo0, clo1, clo2};
+  box_cell(clo, cnx, cny, ncov, t, civ);
+  const int i = civ[0], j = civ[1], k = civ[2];
   const int ii = 2 * i, jj = 2 * j, kk = (LAT::D == 3) ? 2 * k : k;
-  const int nkr = (LAT::D == 3) ? 2 : 1;
+  constexpr int kCh = (LAT::D == 3) ? 8 : 4;
   const double volfrac = (LAT::D == 3) ? 0.125 : 0.25;
-  for (int q = 0; q < LAT::Q; ++q) {
-    double c = 0.0;
-    for (int kr = 0; kr < nkr; ++kr)
-      for (int jr = 0; jr < 2; ++jr)
-        for (int ir = 0; ir < 2; ++ir) c += Ff.at(ii + ir, jj + jr, kk + kr, q);
-    Fc.at(i, j, k, q) = volfrac * c;
-  }
-  for (int n = 0; n < nmac; ++n) {
-    double c = 0.0;
-    for (int kr = 0; kr < nkr; ++kr)
-      for (int jr = 0; jr < 2; ++jr)
-        for (int ir = 0; ir < 2; ++ir) c += Mf.at(ii + ir, jj + jr, kk + kr, n);
-    Mc.at(i, j, k, n) = volfrac * c;
-  }
+  // component blockIdx.y: of f, then of the macros
+  const int n = (int)blockIdx.y;
+  const bool isf = n < LAT::Q;
+  const Fab& S = isf ? Ff : Mf;
+  const Fab& D = isf ? Fc : Mc;
+  const int cn = isf ? n : n - LAT::Q;
+  double v[kCh];
+#pragma unroll
+  for (int u = 0; u < kCh; ++u) v[u] = S.at(ii + (u & 1), jj + ((u >> 1) & 1), kk + (u >> 2), cn);
+  double c = 0.0;
+#pragma unroll
+  for (int u = 0; u < kCh; ++u) c += v[u];
+  D.at(i, j, k, cn) = volfrac * c;
 }
 
 // the coarse cells a fine region's interpolation reads (its parents grown by 1)
@@ -823,9 +1284,9 @@ static void check_coarse_cover(const ilbm_fab* crse, int ncomp, int dim, const i
 
 extern "C" {
 
-int ilbm_box_cf_fill(const ilbm_case_desc* d, const ilbm_fab* crse_old, const ilbm_fab* crse_new, double t_old,
-                     double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine, int ncomp,
-                     const int valid_lo[3], const int valid_hi[3], void* stream) {
+static int box_cf_fill(const ilbm_case_desc* d, const ilbm_fab* crse_old, const ilbm_fab* crse_new, double t_old,
+                       double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine, const ilbm_fab* macro_src,
+                       int ncomp, const int valid_lo[3], const int valid_hi[3], void* stream) {
   if (!d || !valid_lo || !valid_hi || (!f_fine && !macro_fine)) return ILBM_ERR_INVALID;
   if (ncomp < (f_fine ? 4 : 1) || ncomp > ilbm::kMaxInterpComp) return ILBM_ERR_INVALID;
   return guarded([&] {
@@ -840,6 +1301,11 @@ int ilbm_box_cf_fill(const ilbm_case_desc* d, const ilbm_fab* crse_old, const il
         if (macro_fine->lo[e] > domf->lo[e] || macro_fine->hi[e] < domf->hi[e])
           throw StatusError{ILBM_ERR_INVALID, "macro fab does not cover the f fab"};
     }
+    if (macro_src) {
+      check_fab(macro_src, ncomp, G, 0);
+      if (!macro_fine || macro_src->p == macro_fine->p)
+        throw StatusError{ILBM_ERR_INVALID, "macro source without another fab to copy to"};
+    }
     // the fine ghost cells are coarse-fine ghosts: inside the level's domain
     for (int e = 0; e < dim; ++e)
       if (domf->lo[e] < 0 || domf->hi[e] > d->n[e] - 1)
@@ -849,14 +1315,40 @@ int ilbm_box_cf_fill(const ilbm_case_desc* d, const ilbm_fab* crse_old, const il
     const Fab Co = to_fab(*crse_old), Cn = to_fab(*crse_new), D = to_fab(*domf);
     const Fab M = macro_fine ? to_fab(*macro_fine) : Fab{};
     const Fab Fq = f_fine ? to_fab(*f_fine) : Fab{};
+    const Fab Ms = macro_src ? to_fab(*macro_src) : Fab{};
     const TimeMix tm = time_mix(t_old, t_new, time);
+    // in 2D a fab may hold more than the plane the valid box lies in
+    int blo[3], bhi[3];
+    for (int e = 0; e < 3; ++e) {
+      blo[e] = (e < dim) ? G.vlo[e] : D.lo[e];
+      bhi[e] = (e < dim) ? G.vhi[e] : D.hi[e];
+    }
+    const GhostBox gh = ghost_box(D, blo, bhi);
+    const unsigned ng = grid_for(gh.off[6]).x, nv = macro_src ? grid_for(box_cells(G)).x : 0u;
+    if (ng + nv == 0) return;
     with_lattice(box_lattice(*d), [&](auto L) {
       using LAT = decltype(L);
-      hipLaunchKernelGGL(k_box_cf_fill<LAT>, grid_for(D.cells), dim3(256), 0, (hipStream_t)stream, Co, Cn, tm, M, Fq,
-                         D, ncomp, G, 1);
+      hipLaunchKernelGGL(k_box_cf_ghosts<LAT>, dim3(ng + nv), dim3(256), 0, (hipStream_t)stream, Co, Cn, tm, M, Fq, Ms,
+                         ncomp, G, gh, ng);
     });
     HIPCHK(hipGetLastError());
   });
+}
+
+int ilbm_box_cf_fill(const ilbm_case_desc* d, const ilbm_fab* crse_old, const ilbm_fab* crse_new, double t_old,
+                     double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine, int ncomp,
+                     const int valid_lo[3], const int valid_hi[3], void* stream) {
+  return box_cf_fill(d, crse_old, crse_new, t_old, t_new, time, f_fine, macro_fine, nullptr, ncomp, valid_lo, valid_hi,
+                     stream);
+}
+
+int ilbm_box_cf_fill_patch(const ilbm_case_desc* d, const ilbm_fab* crse_old, const ilbm_fab* crse_new, double t_old,
+                           double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine,
+                           const ilbm_fab* macro_src, int ncomp, const int valid_lo[3], const int valid_hi[3],
+                           void* stream) {
+  if (!macro_src) return ILBM_ERR_INVALID;
+  return box_cf_fill(d, crse_old, crse_new, t_old, t_new, time, f_fine, macro_fine, macro_src, ncomp, valid_lo,
+                     valid_hi, stream);
 }
 
 int ilbm_box_interp_from_coarse(const ilbm_case_desc* d, const ilbm_fab* crse, ilbm_fab* macro_fine, int ncomp,
@@ -872,11 +1364,11 @@ int ilbm_box_interp_from_coarse(const ilbm_case_desc* d, const ilbm_fab* crse, i
       if (lo[e] < 0 || hi[e] > d->n[e] - 1) throw StatusError{ILBM_ERR_INVALID, "box outside the level's domain"};
     check_coarse_cover(crse, ncomp, dim, G.vlo, G.vhi);
     const Fab C = to_fab(*crse), M = to_fab(*macro_fine);
-    const TimeMix tm{1, 0.0, 0.0};
+    BoxGeom GV = G;   // in 2D every plane of the fab
+    if (dim == 2) { GV.vlo[2] = M.lo[2]; GV.vhi[2] = M.hi[2]; }
     with_lattice(box_lattice(*d), [&](auto L) {
       using LAT = decltype(L);
-      hipLaunchKernelGGL(k_box_cf_fill<LAT>, grid_for(M.cells), dim3(256), 0, (hipStream_t)stream, C, C, tm, M, Fab{},
-                         M, ncomp, G, 0);
+      hipLaunchKernelGGL(k_box_cf_valid<LAT>, grid_for(box_cells(GV)), dim3(256), 0, (hipStream_t)stream, C, M, ncomp, GV);
     });
     HIPCHK(hipGetLastError());
   });
@@ -907,7 +1399,8 @@ int ilbm_box_average_down(const ilbm_case_desc* d, const ilbm_fab* f_fine, const
     const int64_t ncov = (int64_t)cnx * cny * (chi[2] - clo[2] + 1);
     with_lattice(box_lattice(*d), [&](auto L) {
       using LAT = decltype(L);
-      hipLaunchKernelGGL(k_box_average_down<LAT>, grid_for(ncov), dim3(256), 0, (hipStream_t)stream, to_fab(*f_fine),
+      hipLaunchKernelGGL(k_box_average_down<LAT>, dim3(grid_for(ncov).x, (unsigned)(LAT::Q + nmac)), dim3(256), 0,
+                         (hipStream_t)stream, to_fab(*f_fine),
                          to_fab(*macro_fine), to_fab(*f_crse), to_fab(*macro_crse), nmac, clo[0], clo[1], clo[2], cnx,
                          cny, ncov);
     });

@@ -176,6 +176,12 @@ def load():
     L.ilbm_box_fill_periodic.argtypes = [P(CaseDesc), PF, P(C.c_int), P(C.c_int), vp]
     L.ilbm_box_fill_physical.argtypes = [P(CaseDesc), PF, C.c_int, vp]
     L.ilbm_box_collide.argtypes = [P(CaseDesc), PF, PF, PF, P(C.c_int), P(C.c_int), vp]
+    L.ilbm_box_fill_patch.argtypes = [P(CaseDesc), PF, PF, C.c_int, P(C.c_int), P(C.c_int), vp]
+    L.ilbm_box_fill_collide.argtypes = [P(CaseDesc), PF, PF, PF, PF, C.c_int, P(C.c_int), P(C.c_int), vp]
+    L.ilbm_box_sums_workspace.argtypes = [P(C.c_int), P(C.c_int), C.c_int, P(C.c_int64)]
+    L.ilbm_box_sums.argtypes = [PF, C.c_int, C.c_int, P(C.c_int), P(C.c_int), vp, C.c_int64, P(C.c_double), vp]
+    L.ilbm_box_cf_fill_patch.argtypes = [P(CaseDesc), PF, PF, C.c_double, C.c_double, C.c_double, PF, PF, PF, C.c_int,
+                                         P(C.c_int), P(C.c_int), vp]
     L.ilbm_box_bounce_back.argtypes = [P(CaseDesc), PF, P(C.c_int), P(C.c_int), vp]
     L.ilbm_box_stream_macro.argtypes = [P(CaseDesc), PF, PF, PF, PF, P(C.c_int), P(C.c_int), vp]
     L.ilbm_box_derived.argtypes = [P(CaseDesc), PF, PF, P(C.c_int), P(C.c_int), vp]

@@ -312,6 +312,20 @@ int ilbm_box_fill_physical(const ilbm_case_desc* desc, ilbm_fab* fab, int mesosc
  * (Source/LBM/collide_forced.H:10-51, AdvanceLBMAtLevel.cpp:196-240) */
 int ilbm_box_collide(const ilbm_case_desc* desc, ilbm_fab* f, const ilbm_fab* macro,
                      const ilbm_fab* force, const int valid_lo[3], const int valid_hi[3], void* stream);
+/* FillPatchSingleLevel of a level of one box in one pass: every cell of dst
+ * gets src's valid cell, its periodic image, the physical ghost value of
+ * ilbm_box_fill_physical, or 0.  dst's components are filled (mesoscopic:
+ * at least q); src has at least as many.  The same values as
+ * ilbm_box_setval(0), ilbm_box_copy, ilbm_box_fill_periodic and
+ * ilbm_box_fill_physical in this order. */
+int ilbm_box_fill_patch(const ilbm_case_desc* desc, const ilbm_fab* src, ilbm_fab* dst, int mesoscopic,
+                        const int valid_lo[3], const int valid_hi[3], void* stream);
+/* ilbm_box_fill_patch (mesoscopic) of src into dst, ilbm_box_collide of dst
+ * and ilbm_box_fill_periodic of dst in one pass; with ghosts == 0 only dst's
+ * valid cells are written. */
+int ilbm_box_fill_collide(const ilbm_case_desc* desc, const ilbm_fab* src, ilbm_fab* dst, const ilbm_fab* macro,
+                          const ilbm_fab* force, int ghosts, const int valid_lo[3], const int valid_hi[3],
+                          void* stream);
 /* halfway bounce-back into the user_1 ghost cells (AdvanceLBMAtLevel.cpp:265-373) */
 int ilbm_box_bounce_back(const ilbm_case_desc* desc, ilbm_fab* f, const int valid_lo[3],
                          const int valid_hi[3], void* stream);
@@ -341,6 +355,12 @@ int ilbm_device_synchronize(void);
  * the force integral of ComputeIBForce), fixed order; synchronizes */
 int ilbm_box_sum(const ilbm_fab* fab, int comp, const int lo[3], const int hi[3], double* host_out,
                  void* stream);
+/* ilbm_box_sum of components [comp, comp + ncomp) with one launch of each
+ * kernel, in a workspace of the caller (ilbm_box_sums_workspace bytes of
+ * device memory); the same bits.  Synchronizes. */
+int ilbm_box_sums_workspace(const int lo[3], const int hi[3], int ncomp, int64_t* bytes);
+int ilbm_box_sums(const ilbm_fab* fab, int comp, int ncomp, const int lo[3], const int hi[3], void* work,
+                  int64_t work_bytes, double* host_out, void* stream);
 /* ------------------------------------------------------------------------
  * Coarse-fine transfer between two levels at refinement ratio 2, on
  * caller-owned fabs (level indices; the fine box keeps its ghost cells
@@ -357,6 +377,12 @@ int ilbm_box_sum(const ilbm_fab* fab, int comp, const int lo[3], const int hi[3]
 int ilbm_box_cf_fill(const ilbm_case_desc* desc, const ilbm_fab* crse_old, const ilbm_fab* crse_new, double t_old,
                      double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine, int ncomp,
                      const int valid_lo[3], const int valid_hi[3], void* stream);
+/* ilbm_box_cf_fill that also copies the macros of the valid cells from
+ * macro_src (the level's own macros) to macro_fine */
+int ilbm_box_cf_fill_patch(const ilbm_case_desc* desc, const ilbm_fab* crse_old, const ilbm_fab* crse_new,
+                           double t_old, double t_new, double time, ilbm_fab* f_fine, ilbm_fab* macro_fine,
+                           const ilbm_fab* macro_src, int ncomp, const int valid_lo[3], const int valid_hi[3],
+                           void* stream);
 /* InterpFromCoarseLevel of MakeNewLevelFromCoarse / FillCoarsePatchMacro
  * (AmrCoreLBM.cpp:751-830, 2214-2237): cell_cons_interp of crse over the
  * fine cells [lo, hi] */
