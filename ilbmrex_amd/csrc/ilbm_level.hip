@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -21,6 +22,8 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "ilbm.h"
@@ -60,6 +63,85 @@ static void dev_free(void* p) {
 }
 
 static constexpr double kPi = 3.14159265358979323846;
+
+// Device-to-host copies of whole fields into a caller's ordinary memory.
+// hipMemcpy stages such a copy through one buffer and one core, and the
+// destination is usually fresh memory whose pages the copy touches first
+// (134 MB of macros: 14 ms, 10 GB/s).  Here up to kWorkers threads each own a
+// pinned buffer: a thread queues the transfer of its next slice, waits for it
+// and copies it out, so that transfers run behind each other while the cores
+// share the page faults and the copying: 134 MB in 3.3 ms, 537 MB 51 -> 11.8
+// ms (45 GB/s).  The buffers live with the level (allocated by its first
+// large copy in 2.3 ms, given back with it); copies below kDirect bytes
+// (1.8 ms plain), and any for which no thread can be had, are plain.
+struct HostCopy {
+  static constexpr int kWorkers = 8;
+  static constexpr size_t kSlice = (size_t)4 << 20;
+  static constexpr size_t kDirect = (size_t)32 << 20;
+  char* pinned = nullptr;
+  hipEvent_t ev[kWorkers] = {};
+
+  HostCopy() = default;
+  HostCopy(const HostCopy&) = delete;
+  HostCopy& operator=(const HostCopy&) = delete;
+  ~HostCopy() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (pinned) (void)hipHostFree(pinned);
+  }
+
+  // ordered behind the work of stream s; returns when dst is complete
+  void copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes < kDirect || !ready()) {
+      HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+      HIPCHK(hipStreamSynchronize(s));
+      return;
+    }
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    const size_t slices = (bytes + kSlice - 1) / kSlice;
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto work = [&](int w) {
+      hipError_t e = hipSetDevice(dev);
+      char* buf = pinned + (size_t)w * kSlice;
+      while (e == hipSuccess) {
+        const size_t i = next.fetch_add(1);
+        if (i >= slices) return;
+        const size_t off = i * kSlice, n = std::min(kSlice, bytes - off);
+        e = hipMemcpyAsync(buf, static_cast<const char*>(src) + off, n, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(ev[w], s);
+        if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
+        if (e == hipSuccess) std::memcpy(static_cast<char*>(dst) + off, buf, n);
+      }
+      failed = (int)e;
+    };
+    std::thread th[kWorkers];
+    const int want = (int)std::min<size_t>(kWorkers, slices);
+    for (int w = 1; w < want; ++w) {
+      try {
+        th[w] = std::thread(work, w);
+      } catch (const std::system_error&) {
+        break;   // the threads there are take every slice
+      }
+    }
+    work(0);
+    for (std::thread& t : th)
+      if (t.joinable()) t.join();
+    HIPCHK((hipError_t)failed.load());
+  }
+
+ private:
+  bool ready() {
+    if (pinned) return true;
+    for (hipEvent_t& e : ev)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kWorkers * kSlice, hipHostMallocDefault) != hipSuccess) return false;
+    pinned = static_cast<char*>(p);
+    return true;
+  }
+};
 
 // ---------------------------------------------------------------------------
 // Marker geometry on the host (IBMarkerDF::build_markers,
@@ -488,6 +570,13 @@ static int64_t plane_stride(int64_t cells, int64_t pop_bytes) {
 constexpr int kFarBlocksPerCu = 0;
 constexpr int kFarAfter = 0;
 constexpr int kRingStream = 0;   // Level::RING_NEAR
+// Population bytes of a step from which an IB level overlaps its far cells.
+// Sphere steps in us, overlapped / on one stream: 161x101x99 FP64 (489 MB)
+// 133 / 146, FP32 (245 MB) 78 / 72, FP16-shifted 62 / 53; 192x112x112 FP64
+// 167 / 183, FP32 (366 MB) 89 / 90, FP16-shifted (183 MB) 58 / 59;
+// 256x128x128 FP32 (637 MB) 122 / 125, FP16-shifted (319 MB) 77 / 75.
+// ILBM_OVERLAP_BYTES overrides it.
+constexpr int64_t kOverlapBytes = (int64_t)350 << 20;
 
 // Dynamic LDS a body tile may take: the stream-collide blocks of the launch
 // get it too (8 blocks of 256 threads fill a CU).
@@ -580,6 +669,7 @@ struct Level {
   double* mout = nullptr;
   double* fout = nullptr;
   bool state_valid = false;
+  HostCopy host_copy;
   // histories
   double* mass_dev = nullptr;
   int mass_cap = 0;
@@ -1763,6 +1853,11 @@ struct Level {
     // below ~1M cells the two cross-stream waits per step cost more than
     // the overlap saves (512x256 D2Q9 FP64: 2.5 -> 1.9 GLUPS with it)
     if (ncells < ((int64_t)1 << 20)) return false;
+    // and so they do where the far cells' launch is shorter than the host
+    // needs to queue an overlapped step (60-75 us): under kOverlapBytes of
+    // populations read and written per step
+    const char* ob = std::getenv("ILBM_OVERLAP_BYTES");
+    if (ncells * 2 * c.q * (int64_t)popbytes < (ob ? (int64_t)std::atoll(ob) : kOverlapBytes)) return false;
     if (!stream_b) {
       int per_cu = kFarBlocksPerCu;
       if (const char* e = std::getenv("ILBM_FAR_BLOCKS_PER_CU")) per_cu = std::max(0, std::atoi(e));
@@ -2351,7 +2446,7 @@ int ilbm_level_get_f(ilbm_level* h, double* out) {
   if (!h || !out) return ILBM_ERR_INVALID;
   if (!h->L.state_valid) return ILBM_ERR_STATE;
   return guarded([&] {
-    HIPCHK(hipMemcpy(out, h->L.fout, sizeof(double) * h->L.c.q * h->L.ncells, hipMemcpyDeviceToHost));
+    h->L.host_copy.copy(out, h->L.fout, sizeof(double) * h->L.c.q * h->L.ncells, h->L.stream);
   });
 }
 
@@ -2359,7 +2454,7 @@ int ilbm_level_get_macro(ilbm_level* h, double* out) {
   if (!h || !out) return ILBM_ERR_INVALID;
   if (!h->L.state_valid) return ILBM_ERR_STATE;
   return guarded([&] {
-    HIPCHK(hipMemcpy(out, h->L.mout, sizeof(double) * 4 * h->L.ncells, hipMemcpyDeviceToHost));
+    h->L.host_copy.copy(out, h->L.mout, sizeof(double) * 4 * h->L.ncells, h->L.stream);
   });
 }
 
