@@ -1486,7 +1486,7 @@ __global__ void __launch_bounds__(kSumsBlock) k_ghosts_record(GhostArgs g, unsig
 // 112.1 against 107.4 us).  The block (k_step's shape) holds kSumsBlock
 // threads and the record's reductions number them linearly, so its tree is
 // k_sums_record's.
-template <class LAT, class ST, int AM>
+template <class LAT, class ST, int AM, bool LIN = false>
 __global__ void __launch_bounds__(kBlock) k_step_record(StepArgs a, uint32_t tx, uint32_t ty, uint32_t ntiles,
                                                         IbArgs ia, RecArgs rec, int nblk) {
   (void)ntiles;
@@ -1496,6 +1496,10 @@ __global__ void __launch_bounds__(kBlock) k_step_record(StepArgs a, uint32_t tx,
   }
   const uint32_t t = blockIdx.x - 1;
   __shared__ double lds[kBlock / 64];
+  if constexpr (LIN) {
+    step_lin_body<LAT, ST, AM>(a, t, lds);
+    return;
+  }
   const uint32_t bz = t / (tx * ty), rem = t - bz * tx * ty, by = rem / tx, bx = rem - by * tx;
   const int o0 = (a.sub_mode >= 2) ? a.sub_lo[0] : 0, o1 = (a.sub_mode >= 2) ? a.sub_lo[1] : 0;
   const int o2 = (a.sub_mode >= 2) ? a.sub_lo[2] : 0;

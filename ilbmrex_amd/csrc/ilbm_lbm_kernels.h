@@ -157,6 +157,18 @@ __host__ __device__ inline int64_t slab_index(const Slabs& S, const int c[3], in
 // boundary condition types (AMReX BCType and the reference's user kinds)
 enum { BC_INT_DIR = 0, BC_FOEXTRAP = 2, BC_EXT_DIR = 3, BC_USER_1 = 1001, BC_USER_2 = 1002 };
 
+// n / d for n < 2^31 as a multiply and a shift: mul = floor(2^(31 + l) / d) + 1
+// with l = ceil(log2 d) is exact for such n
+struct FastDiv {
+  uint32_t mul, sh;
+  __device__ uint32_t operator()(uint32_t n) const { return (uint32_t)(((uint64_t)n * mul) >> sh); }
+};
+inline FastDiv fast_div(uint32_t d) {
+  uint32_t l = 0;
+  while (((uint64_t)1 << l) < d) ++l;
+  return FastDiv{(uint32_t)((((uint64_t)1 << (31 + l)) / d) + 1), 31 + l};
+}
+
 struct StepArgs {
   GridGeom g;
   Slabs slabs;
@@ -197,6 +209,10 @@ struct StepArgs {
   // other cells (0, unless rho is not finite), null where none follows
   double* Fnext;
   double dt;
+  // lin: the launch's blocks hold 256 consecutive elements each of the
+  // level's stored rows (step_lin_body); div_x by the row stride, div_y by n[1]
+  int lin;
+  FastDiv div_x, div_y;
   // the uniform parameters rounded once to FP32 on the host, for shifted
   // storage (bound by vector ALU issue: no per-wavefront conversion or
   // divide): (float)tau, (float)inv_tau, 1 - 0.5 / (float)tau, (float)Fmac,
@@ -910,9 +926,31 @@ __device__ __forceinline__ void step_body_masked(const StepArgs& a, bool on, int
 // instructions per wavefront).
 __device__ __forceinline__ int wave_row(int j) { return __builtin_amdgcn_readfirstlane(j); }
 
+// Cell of thread t of block blk of a linear launch: 256 consecutive elements
+// of the rows as they are stored, padding included, so that a wavefront's
+// loads and stores stay whole cache lines.  Rows stored in an odd number of
+// 32-cell pieces leave half a wavefront (or more) of the row tiling idle on
+// every row; here a wavefront runs into the next row instead, for some vector
+// arithmetic that a row's wavefronts keep in scalar registers.  Without the
+// padding every lane has a cell, but lines are then stored in parts: slower
+// than the row tiling at almost every extent.  A thread in the padding or
+// past the last cell gets i >= n[0], inactive.
 template <class LAT, class ST, int AM>
+__device__ __forceinline__ void step_lin_body(const StepArgs& a, uint32_t blk, double* lds) {
+  const uint32_t c = blk * (uint32_t)kBlock + threadIdx.x;
+  const uint32_t row = a.div_x(c), pl = a.div_y(row);
+  const int i = (int)(c - row * (uint32_t)a.g.js), j = (int)(row - pl * (uint32_t)a.g.n[1]), k = (int)pl;
+  step_body<LAT, ST, AM>(a, (k < a.g.n[2]) ? i : a.g.n[0], j, k, (int64_t)blk, lds);
+}
+
+// LIN: a linear launch (3D lattices)
+template <class LAT, class ST, int AM, bool LIN = false>
 __global__ void __launch_bounds__(kBlock) k_step(StepArgs a) {
   __shared__ double lds[kBlock / 64];
+  if constexpr (LIN) {
+    step_lin_body<LAT, ST, AM>(a, blockIdx.x, lds);
+    return;
+  }
   const int64_t blk = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
   const int o0 = (a.sub_mode >= 2) ? a.sub_lo[0] : 0, o1 = (a.sub_mode >= 2) ? a.sub_lo[1] : 0;
   const int o2 = (a.sub_mode >= 2) ? a.sub_lo[2] : 0;

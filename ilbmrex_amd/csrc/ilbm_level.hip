@@ -406,6 +406,13 @@ template <class LAT, class ST, int AM>
 static void launch_step(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, hipEvent_t e0, hipEvent_t e1) {
   check_step_block(b);
   const uint32_t nt = g.x * g.y * g.z;
+  if constexpr (LAT::D == 3) {
+    if (a.lin && a.sub_mode < 2) {   // 256 x 1 blocks
+      if (e0) hipExtLaunchKernelGGL((k_step<LAT, ST, AM, true>), g, b, 0, s, e0, e1, 0, a);
+      else hipLaunchKernelGGL((k_step<LAT, ST, AM, true>), g, b, 0, s, a);
+      return;
+    }
+  }
   if (a.persist > 0 && nt > (uint32_t)a.persist) {
     const dim3 pg((unsigned)a.persist);
     if (e0) hipExtLaunchKernelGGL((k_step_p<LAT, ST, AM>), pg, b, 0, s, e0, e1, 0, a, g.x, g.y, nt);
@@ -449,6 +456,12 @@ static void launch_step_rec(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, co
                             int nblk) {
   check_step_block(b);
   const uint32_t nt = g.x * g.y * g.z;
+  if constexpr (LAT::D == 3) {
+    if (a.lin) {
+      hipLaunchKernelGGL((k_step_record<LAT, ST, AM, true>), dim3(nt + 1), b, 0, s, a, g.x, g.y, nt, ia, r, nblk);
+      return;
+    }
+  }
   hipLaunchKernelGGL((k_step_record<LAT, ST, AM>), dim3(nt + 1), b, 0, s, a, g.x, g.y, nt, ia, r, nblk);
 }
 
@@ -578,6 +591,10 @@ constexpr int kRingStream = 0;   // Level::RING_NEAR
 // ILBM_OVERLAP_BYTES overrides it.
 constexpr int64_t kOverlapBytes = (int64_t)350 << 20;
 
+// FP32 and FP64 levels from this many cells may step in linear blocks
+// (Level::linear_steps).
+constexpr int64_t kLinCells = (int64_t)3 << 20;
+
 // Dynamic LDS a body tile may take: the stream-collide blocks of the launch
 // get it too (8 blocks of 256 threads fill a CU).
 constexpr int kBodyLds = 20 * 1024;
@@ -606,6 +623,11 @@ struct Level {
   double* partial = nullptr;
   int64_t nblocks = 0;
   dim3 grid, block;
+  // the launches of a level that steps on its own: the row tiling above, or
+  // linear blocks (step_lin)
+  bool step_lin = false;
+  int64_t step_nblk = 0;
+  dim3 step_grid, step_block;
   StepFn stepfn = nullptr;
   InitFn initfn = nullptr;
   FixFn fixfn = nullptr;
@@ -936,7 +958,11 @@ struct Level {
     block = dim3(bx, by, 1);
     grid = dim3((c.n[0] + bx - 1) / bx, (c.n[1] + by - 1) / by, c.n[2]);
     nblocks = (int64_t)grid.x * grid.y * grid.z;
-    ensure_partial(nblocks);
+    step_lin = linear_steps();
+    step_nblk = step_lin ? (g.js * c.n[1] * c.n[2] + kBlock - 1) / kBlock : nblocks;
+    step_grid = step_lin ? dim3((unsigned)step_nblk) : grid;
+    step_block = step_lin ? dim3(kBlock) : block;
+    ensure_partial(std::max(nblocks, step_nblk));
     clock_d = dev_alloc<double>(4);
 
     auto pk = [&](auto latt) {
@@ -953,6 +979,24 @@ struct Level {
     else pick_body<StF16S>(lat, am, stepbodyfn, bodyfn);
     tau = 3.0 * c.nu / c.dx[0] + 0.5;  // AmrCoreLBM.cpp:225
     dt = c.dx[0];                       // AmrCoreLBM.cpp:228
+  }
+
+  // Whether the level's own steps run in linear blocks (ILBM_STEP_LINEAR=0 /
+  // 1 decides otherwise): 3D levels whose stored rows are an odd number of
+  // 32-cell pieces, so that the row tiling (a wavefront per 64 cells of a
+  // row) idles at least half a wavefront per row -- in FP16-shifted storage,
+  // whose kernel is bound by instruction issue, at any size; in FP32 and FP64
+  // on rows of one piece and on large levels.  k_step in us, rows -> linear:
+  // FP16-shifted 160^3 77 -> 62, 200x160x160 sphere 100 -> 88, 96^3 18.4 ->
+  // 15.8 (rows of whole wavefronts lose: duct 48x112x112 19.1 -> 22.1); duct
+  // 24x96x96 FP64 41.6 -> 29.7, FP16-shifted 14.1 -> 11.4; FP32 160^3 112.5
+  // -> 107.4, 130x160x160 117 -> 110, 145x120x120 65.6 -> 65.8, 90x96x96 29.6
+  // -> 31.1; FP64 200^3 440 -> 423, 150x120x120 126.4 -> 126.7.
+  bool linear_steps() const {
+    if (c.dim != 3 || g.js * c.n[1] * c.n[2] >= ((int64_t)1 << 31) - kBlock) return false;
+    if (const char* e = std::getenv("ILBM_STEP_LINEAR")) return e[0] == '1';
+    if (g.js % 64 == 0) return false;
+    return st == 2 || g.js <= 32 || ncells >= kLinCells;
   }
 
   // number of blocks of a tile of width bx (height kBlock / bx)
@@ -1690,6 +1734,8 @@ struct Level {
     a.tile_bx = (int)block.x;
     a.tile_nc = 1;
     a.persist = 0;
+    a.div_x = fast_div((uint32_t)g.js);
+    a.div_y = fast_div((uint32_t)c.n[1]);
     a.off32 = ((int64_t)popbytes * g.pop_n < ((int64_t)1 << 32)) ? 1 : 0;
     a.ftau = (float)a.tau;
     a.finv_tau = (float)a.inv_tau;
@@ -1945,10 +1991,11 @@ struct Level {
   // box.
   void split_step(int s, double time, bool want, bool more) {
     StepArgs sf = step_args(want);
+    sf.lin = step_lin ? 1 : 0;
     sf.sub_mode = 1;
     sf.persist = far_persist;
     for (int d = 0; d < 3; ++d) { sf.sub_lo[d] = near_lo[d]; sf.sub_n[d] = near_n[d]; }
-    sf.partial = mring + (int64_t)mring_used * nblocks;
+    sf.partial = mring + (int64_t)mring_used * step_nblk;
     StepArgs sn = sf;
     sn.persist = 0;
     sn.sub_mode = 2;
@@ -1963,7 +2010,7 @@ struct Level {
       ghost_done = xsignal(stream_b, X_GHOST);
     }
     ghost_ahead = false;
-    stepfn(grid, block, stream_b, sf, nullptr, nullptr);
+    stepfn(step_grid, step_block, stream_b, sf, nullptr, nullptr);
     ring_slot = async_record() ? s % kRecRing : -1;
     ib_update_forcing(time, s);
     ring_slot = -1;
@@ -2006,7 +2053,7 @@ struct Level {
   void flush_mass(hipStream_t st) {
     if (pend.n <= 0) return;
     hipLaunchKernelGGL(k_mass_ring, dim3(pend.n), dim3(1024), 0, st,
-                       (const double*)(mring + (int64_t)pend.base * nblocks), nblocks, nblocks,
+                       (const double*)(mring + (int64_t)pend.base * step_nblk), step_nblk, step_nblk,
                        (const double*)(nring + (int64_t)pend.base * nblocks_near), nblocks_near, nblocks_near,
                        (const double*)(rring + (int64_t)pend.base * nblocks_ring), nblocks_ring, nblocks_ring,
                        mass_dev + pend.s + 1 - pend.n);
@@ -2017,11 +2064,12 @@ struct Level {
 
   void split_step3(int s, double time, bool want, bool more, bool first) {
     StepArgs sf = step_args(want);
+    sf.lin = step_lin ? 1 : 0;
     sf.sub_mode = 1;
     sf.persist = far_persist;
     for (int d = 0; d < 3; ++d) { sf.sub_lo[d] = ring_lo[d]; sf.sub_n[d] = ring_n[d]; }
     const int slot = mring_used;
-    sf.partial = mring + (int64_t)slot * nblocks;
+    sf.partial = mring + (int64_t)slot * step_nblk;
     StepArgs sn = sf;
     sn.persist = 0;
     sn.sub_mode = 2;
@@ -2052,7 +2100,7 @@ struct Level {
       if (!ghost_ahead && npad && !slabs_fresh) ghostfn(ggrid, dim3(kGhostBlock), stream_b, ghost_args());
       ghost_ahead = false;
       if (far_after) xwait(stream_b, X_IB, ib_sig);
-      stepfn(grid, block, stream_b, sf, nullptr, nullptr);
+      stepfn(step_grid, step_block, stream_b, sf, nullptr, nullptr);
       far_sig[s & 1] = xsignal(stream_b, X_FAR0 + (s & 1));
       if (more && npad && !gfuse) {
         cur ^= 1;
@@ -2099,7 +2147,7 @@ struct Level {
       if (!ghost_ahead && npad && !slabs_fresh) ghostfn(ggrid, dim3(kGhostBlock), stream_b, ghost_args());
       ghost_ahead = false;
       if (far_after) xwait(stream_b, X_IB, ib_sig);
-      stepfn(grid, block, stream_b, sf, nullptr, nullptr);
+      stepfn(step_grid, step_block, stream_b, sf, nullptr, nullptr);
       if (more && npad && !gfuse) {
         cur ^= 1;
         const GhostArgs ga = ghost_args();
@@ -2143,7 +2191,7 @@ struct Level {
     if (!ghost_ahead && npad && !slabs_fresh) ghostfn(ggrid, dim3(kGhostBlock), stream_b, ghost_args());
     ghost_ahead = false;
     if (far_after) xwait(stream_b, X_IB, ib_sig);
-    stepfn(grid, block, stream_b, sf, nullptr, nullptr);
+    stepfn(step_grid, step_block, stream_b, sf, nullptr, nullptr);
     far_sig[s & 1] = xsignal(stream_b, X_FAR0 + (s & 1));
     if (more && npad && !gfuse) {
       cur ^= 1;
@@ -2184,8 +2232,8 @@ struct Level {
     const int n = mring_used - mring_base;
     if (n == mring_slots / 2 || !more) {
       const bool with_ring = with_near && rring;
-      hipLaunchKernelGGL(k_mass_ring, dim3(n), dim3(1024), 0, st, (const double*)(mring + (int64_t)mring_base * nblocks),
-                         nblocks, nblocks, (const double*)(with_near ? nring + (int64_t)mring_base * nblocks_near : nullptr),
+      hipLaunchKernelGGL(k_mass_ring, dim3(n), dim3(1024), 0, st, (const double*)(mring + (int64_t)mring_base * step_nblk),
+                         step_nblk, step_nblk, (const double*)(with_near ? nring + (int64_t)mring_base * nblocks_near : nullptr),
                          with_near ? nblocks_near : (int64_t)0, with_near ? nblocks_near : (int64_t)0,
                          (const double*)(with_ring ? rring + (int64_t)mring_base * nblocks_ring : nullptr),
                          with_ring ? nblocks_ring : (int64_t)0, with_ring ? nblocks_ring : (int64_t)0,
@@ -2209,13 +2257,13 @@ struct Level {
   // ring slots for the mass partials of this level (and its near box)
   void ensure_mring(bool split) {
     const bool three = split && ring_ok;
-    const int64_t per = nblocks + (split ? nblocks_near : 0) + (three ? nblocks_ring : 0);
+    const int64_t per = step_nblk + (split ? nblocks_near : 0) + (three ? nblocks_ring : 0);
     if (mring && (!split || nring) && (!three || rring)) return;
     dev_free(mring); dev_free(nring); dev_free(rring);
     mring = nring = rring = nullptr;
     // two halves of at most 32 steps each, at most 64 MiB
     mring_slots = 2 * (int)std::max<int64_t>(1, std::min<int64_t>(32, ((int64_t)32 << 20) / (8 * per)));
-    mring = dev_alloc<double>((size_t)nblocks * mring_slots);
+    mring = dev_alloc<double>((size_t)step_nblk * mring_slots);
     if (split) nring = dev_alloc<double>((size_t)nblocks_near * mring_slots);
     if (three) rring = dev_alloc<double>((size_t)nblocks_ring * mring_slots);
     mring_used = mring_base = 0;
@@ -2278,20 +2326,21 @@ struct Level {
       }
       // a record still held goes with the stream-collide launch as its last
       // block, unless the launch is timed (then on its own, before it)
-      const bool rec_with_step = rec_held && !timing && block.x * block.y == (unsigned)kSumsBlock;
+      const bool rec_with_step = rec_held && !timing && step_block.x * step_block.y == (unsigned)kSumsBlock;
       if (rec_held && !rec_with_step) {
         hipLaunchKernelGGL(k_sums_record, dim3(1), dim3(kSumsBlock), 0, stream, held_a, held_r, held_nblk);
         rec_held = false;
       }
       const bool last = (s == nsteps - 1);
       StepArgs sa = step_args(want_state && last);
-      sa.partial = mring + (int64_t)mring_used * nblocks;
+      sa.lin = step_lin ? 1 : 0;
+      sa.partial = mring + (int64_t)mring_used * step_nblk;
       if (rec_with_step) {
-        steprecfn(grid, block, stream, sa, held_a, held_r, held_nblk);
+        steprecfn(step_grid, step_block, stream, sa, held_a, held_r, held_nblk);
         rec_held = false;
       } else {
         // timing: the dispatch records the kernel's own begin / end
-        stepfn(grid, block, stream, sa, timing ? ev_start[s] : nullptr, timing ? ev_stop[s] : nullptr);
+        stepfn(step_grid, step_block, stream, sa, timing ? ev_start[s] : nullptr, timing ? ev_stop[s] : nullptr);
       }
       ring_step(stream, s, !last, false);
       slabs_fresh = gfuse;
@@ -2587,7 +2636,7 @@ int ilbm_level_info(ilbm_level* h, double out[8]) {
   out[4] = (double)L.band_cells; out[5] = (double)L.popbytes;
   out[6] = (L.am == ilbm::kAddrWrap) ? 0.0 : (L.am == ilbm::kAddrWall64) ? 1.0 : (L.am == ilbm::kAddrWall32) ? 2.0
            : L.gfuse ? 4.0 : 3.0;
-  out[7] = (double)L.nblocks;
+  out[7] = (double)L.step_nblk;
   return ILBM_OK;
 }
 
