@@ -44,12 +44,64 @@ template <class LAT, class ST>
 __global__ void __launch_bounds__(kBlock) k_cf_fill_move(CfArgs a, unsigned ncf, MoveArgs mv, IbArgs ia) {
   static_assert(kBlock == 256, "ghost and marker blocks share the launch's block size");
   if (blockIdx.x < ncf) cf_fill_body<LAT, ST>(a, (int64_t)blockIdx.x * kBlock + threadIdx.x);
-  else move_weights_body(mv, ia, (int)(blockIdx.x - ncf));
+  else move_weights_body(mv, ia, (int)((blockIdx.x - ncf) * kBlock + threadIdx.x));
 }
 template <class LAT, class ST>
 static void launch_cf_move(unsigned ncf, unsigned nmv, hipStream_t s, const CfArgs& a, const MoveArgs& mv,
                            const IbArgs& ia) {
   hipLaunchKernelGGL((k_cf_fill_move<LAT, ST>), dim3(ncf + nmv), dim3(kBlock), 0, s, a, ncf, mv, ia);
+}
+
+// A 2D level's stream-collide with the coarse-fine fills of the sub-steps
+// after it in its first blocks: of the level's own second sub-step (into the
+// buffer the step writes, whose slabs it leaves alone) and of the finer
+// level's first (whose window is at its old state), each with that level's
+// marker kinematics where its body moves.  The step reads and writes none of
+// their data.  The levels of a 2D hierarchy step in about 5 us, so it is the
+// chain of launches that a coarse step waits for: alone, a fill takes 6 us
+// and one with kinematics 7.3; beside the step they end with it.
+struct CfRide {
+  unsigned n[2], nmv;   // blocks of each fill, of the kinematics
+  CfArgs cf[2];
+  MoveArgs mv;
+  IbArgs ib;
+};
+template <class LAT, class ST, int AM>
+__global__ void __launch_bounds__(kBlock) k_step_cf(StepArgs a, uint32_t tx, CfRide r) {
+  static_assert(LAT::D == 2, "2D levels");
+  __shared__ double lds[kBlock / 64];
+  uint32_t b = blockIdx.x;
+  for (int k = 0; k < 2; ++k) {
+    if (b < r.n[k]) {
+      cf_fill_body<LAT, ST>(r.cf[k], (int64_t)b * lin_nt() + lin_tid());
+      return;
+    }
+    b -= r.n[k];
+  }
+  if (b < r.nmv) {
+    move_weights_body(r.mv, r.ib, (int)b * lin_nt() + lin_tid());
+    return;
+  }
+  b -= r.nmv;
+  const uint32_t by = b / tx, bx = b - by * tx;
+  step_body<LAT, ST, AM>(a, (int)(bx * blockDim.x + threadIdx.x), wave_row((int)(by * blockDim.y + threadIdx.y)), 0, b,
+                         lds);
+}
+using StepCfFn = void (*)(dim3, dim3, hipStream_t, const StepArgs&, const CfRide&);
+template <class ST, int AM>
+static void launch_step_cf(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, const CfRide& r) {
+  check_step_block(b);
+  hipLaunchKernelGGL((k_step_cf<D2Q9, ST, AM>), dim3(g.x * g.y + r.n[0] + r.n[1] + r.nmv), b, 0, s, a, g.x, r);
+}
+// none in 3D or for 64-bit offsets
+static StepCfFn pick_step_cf(int lat, int st, int am) {
+  if (lat != 0 || am == kAddrWall64) return nullptr;
+  auto pk = [&](auto stt) -> StepCfFn {
+    using ST = decltype(stt);
+    return (am == kAddrWrap) ? launch_step_cf<ST, kAddrWrap>
+         : (am == kAddrWallX32) ? launch_step_cf<ST, kAddrWallX32> : launch_step_cf<ST, kAddrWall32>;
+  };
+  return st == 0 ? pk(StF64{}) : st == 1 ? pk(StF32{}) : pk(StF16S{});
 }
 
 template <class LAT, class ST>
@@ -70,6 +122,14 @@ static void pick_amr(int lat, int st, CfFn& cf, AvgFn& av, CfMoveFn& cm) {
 }
 
 constexpr int kMaxLev = 3;
+// Levels up to this size take the fills of the next sub-steps with their
+// stream-collide (k_step_cf).  us per coarse step of a cylinder with one
+// refined box, fills apart and taken along, by level-0 cells: 512x256 FP64
+// 75 and 63, FP32 65 and 56, FP16-shifted 66 and 55; 1448x724 104 and 96, 81
+// and 76, 76 and 73; beyond, the registers of the fill cost the step more
+// waves than the launch is worth: 2048x1024 FP32 96 and 98, FP16-shifted 83
+// and 89.
+constexpr int64_t kRideCells = (int64_t)1 << 20;
 
 struct Amr {
   hipStream_t stream = nullptr;
@@ -81,6 +141,8 @@ struct Amr {
   double* dpartial[kMaxLev] = {nullptr, nullptr, nullptr};
   int64_t dblocks[kMaxLev] = {0, 0, 0};
   bool exported[kMaxLev] = {false, false, false};
+  int64_t ride_cells = kRideCells;   // ILBM_AMR_RIDE_CELLS
+  bool cf_ready[kMaxLev] = {false, false, false};   // the next sub-step's fill (and kinematics) went with an earlier launch
   CfFn cffn = nullptr;
   CfMoveFn cfmovefn = nullptr;
   AvgFn avgfn = nullptr;
@@ -233,6 +295,7 @@ struct Amr {
     const Level& F = *L[nlev - 1];
     ncol = F.ib ? F.ncol : 0;
     pick_amr(L[0]->lat, L[0]->st, cffn, avgfn, cfmovefn);
+    if (const char* e = std::getenv("ILBM_AMR_RIDE_CELLS")) ride_cells = std::atoll(e);
     HIPCHK(hipStreamSynchronize(stream));
   }
 
@@ -289,25 +352,67 @@ struct Amr {
     W.b = (time - C.t_old) / (C.t_new - C.t_old);
   }
 
-  // with_move: the level's moving-body kinematics at `time` go in the same
-  // launch (k_cf_fill_move) and its next forcing skips them
-  void cf_fill(int l, double time, bool with_move = false) {
-    Level& V = *L[l];
+  // the fill of level l's ghost slabs in buffer `buf` at `time`
+  CfArgs cf_args(int l, double time, int buf) const {
+    const Level& V = *L[l];
     CfArgs a{};
     a.g = V.g;
     a.slabs = V.slabs;
-    a.gbuf = V.gbuf[V.cur];
+    a.gbuf = V.gbuf[buf];
     for (int d = 0; d < 3; ++d) a.ioff[d] = (d < dim) ? V.ioff[d] : 0;
     a.ncomp = V.c.nmac;
     window_at(l - 1, time, a.W);
-    const int64_t npad = V.slabs.face_off[V.slabs.nface];
-    const unsigned ncf = (unsigned)((npad + kBlock - 1) / kBlock);
-    if (with_move) {
+    return a;
+  }
+  static int64_t cf_cells(const Level& V) { return V.slabs.face_off[V.slabs.nface]; }
+  static bool moves(const Level& V) { return V.ib && V.dev_kin; }
+
+  // with the level's moving-body kinematics at `time` in the same launch
+  // (k_cf_fill_move), which its next forcing then skips
+  void cf_fill(int l, double time) {
+    Level& V = *L[l];
+    if (cf_ready[l]) {
+      cf_ready[l] = false;
+      V.moved_ext = moves(V);
+      return;
+    }
+    const CfArgs a = cf_args(l, time, V.cur);
+    const unsigned ncf = (unsigned)((cf_cells(V) + kBlock - 1) / kBlock);
+    if (moves(V)) {
       cfmovefn(ncf, (unsigned)((V.nm + kBlock - 1) / kBlock), stream, a, V.move_args(time), V.ib_args());
       V.moved_ext = true;
       return;
     }
     cffn(dim3(ncf), stream, a);
+  }
+
+  // The fills that can go with the stream-collide of level l's sub-step at
+  // `time`: its own next one (first: the sub-step is the first of two) and
+  // the finer level's first.  Levels of more than kRideCells cells keep them
+  // apart.
+  bool ride_args(int l, double time, bool first, CfRide& r) {
+    Level& V = *L[l];
+    if (!pick_step_cf(V.lat, V.st, V.am) || V.ncells > ride_cells) return false;
+    const unsigned nt = V.block.x * V.block.y;
+    r = CfRide{};
+    auto add = [&](int k, int m, double t, int buf) {
+      Level& F = *L[m];
+      r.cf[k] = cf_args(m, t, buf);
+      r.n[k] = (unsigned)((cf_cells(F) + nt - 1) / nt);
+      if (moves(F)) {
+        r.mv = F.move_args(t);
+        r.ib = F.ib_args();
+        r.nmv = (unsigned)((F.nm + nt - 1) / nt);
+      }
+      cf_ready[m] = true;
+    };
+    if (first && l > 0) add(0, l, time + V.dt, V.cur ^ 1);
+    if (l < nlev - 1) {
+      Window W{};
+      window_at(l, time, W);
+      if (W.mode == 0) add(1, l + 1, time, L[l + 1]->cur);   // the step writes the new state
+    }
+    return r.n[0] + r.n[1] > 0;
   }
 
   void average_down(int l) {
@@ -646,7 +751,8 @@ struct Amr {
     ++nregrid;
   }
 
-  void substep(int l, double time, bool last_chain, int row, bool export_state) {
+  // first: the first of the two sub-steps of a refined level
+  void substep(int l, double time, bool last_chain, int row, bool export_state, bool first = false) {
     if (regrid_on && l < nlev - 1 && L[l]->istep > last_regrid[l] && L[l]->istep % regrid_int == 0) {
       regrid(l, time);
       for (int k = l; k < nlev; ++k) last_regrid[k] = L[k]->istep;
@@ -664,7 +770,7 @@ struct Amr {
     V.t_old = V.t_new;
     V.t_new += V.dt;
     if (V.window) V.wsel ^= 1;  // swap(macro_new, macro_old)
-    if (l > 0) cf_fill(l, time, V.ib && V.dev_kin);
+    if (l > 0) cf_fill(l, time);
     if (V.ib) {
       V.rec_enable = last_chain;
       V.rec_override = true;
@@ -683,9 +789,12 @@ struct Amr {
                   V.ghost_args());
     }
     StepArgs sa = V.step_args(export_state);
+    CfRide ride;
     if (V.rec_held) {
       V.steprecfn(V.grid, V.block, stream, sa, V.held_a, V.held_r, V.held_nblk);
       V.rec_held = false;
+    } else if (ride_args(l, time, first, ride)) {
+      pick_step_cf(V.lat, V.st, V.am)(V.grid, V.block, stream, sa, ride);
     } else {
       V.stepfn(V.grid, V.block, stream, sa, nullptr, nullptr);
     }
@@ -697,7 +806,7 @@ struct Amr {
     ++V.istep;
     if (l < nlev - 1) {
       for (int i = 1; i <= 2; ++i)
-        substep(l + 1, time + (double)(i - 1) * L[l + 1]->dt, last_chain && i == 2, row, i == 2);
+        substep(l + 1, time + (double)(i - 1) * L[l + 1]->dt, last_chain && i == 2, row, i == 2, i == 1);
       average_down(l);
       derived(l, V.wsel);
     }
@@ -719,6 +828,7 @@ struct Amr {
     for (int s = 0; s < nsteps; ++s) {
       const double time = C0.t_new;
       step_end = time + C0.dt;
+      for (bool& r : cf_ready) r = false;   // (set where an error ended a step)
       substep(0, time, true, s, want_state && s == nsteps - 1);
       ++istep;
       hipLaunchKernelGGL(k_mass_total, dim3(1), dim3(1024), 0, stream, (const double*)C0.partial, C0.nblocks,

@@ -769,9 +769,9 @@ struct MoveArgs {
 // One pass per step of a moving body: positions and target velocities
 // (k_ib_move), stencil cells and weights (k_ib_weights), and the cell bounds
 // of each kMarkerChunk-marker chunk (k_ib_chunk_bounds) from a 32-lane
-// min / max; blocks hold whole chunks.
-__device__ __forceinline__ void move_weights_body(const MoveArgs& mv, const IbArgs& a, int blk) {
-  const int m = blk * (int)blockDim.x + (int)threadIdx.x;
+// min / max; wavefronts hold whole chunks.  m: the thread's marker, also
+// beyond the last.
+__device__ __forceinline__ void move_weights_body(const MoveArgs& mv, const IbArgs& a, int m) {
   const int nm = a.nm;
   const bool act = m < nm;
   int b[3] = {0, 0, 0};
@@ -804,7 +804,9 @@ __device__ __forceinline__ void move_weights_body(const MoveArgs& mv, const IbAr
   }
 }
 
-__global__ void __launch_bounds__(256) k_ib_move_weights(MoveArgs mv, IbArgs a) { move_weights_body(mv, a, blockIdx.x); }
+__global__ void __launch_bounds__(256) k_ib_move_weights(MoveArgs mv, IbArgs a) {
+  move_weights_body(mv, a, (int)(blockIdx.x * blockDim.x + threadIdx.x));
+}
 
 // Block size of the one-block reductions (marker sums, force record): every
 // launch of a level, a batch or a hierarchy uses it, so the trees are the
