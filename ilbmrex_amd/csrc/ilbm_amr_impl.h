@@ -30,7 +30,7 @@ namespace ilbm {
 
 using CfFn = void (*)(dim3, hipStream_t, const CfArgs&);
 using CfMoveFn = void (*)(unsigned, unsigned, hipStream_t, const CfArgs&, const MoveArgs&, const IbArgs&);
-using AvgFn = void (*)(dim3, hipStream_t, const AvgArgs&);
+using AvgFn = void (*)(unsigned, unsigned, hipStream_t, const AvgArgs&, const DerArgs&);
 
 template <class LAT, class ST>
 static void launch_cf(dim3 g, hipStream_t s, const CfArgs& a) {
@@ -105,8 +105,8 @@ static StepCfFn pick_step_cf(int lat, int st, int am) {
 }
 
 template <class LAT, class ST>
-static void launch_avg(dim3 g, hipStream_t s, const AvgArgs& a) {
-  hipLaunchKernelGGL((k_average_down<LAT, ST>), g, dim3(256), 0, s, a);
+static void launch_avg(unsigned navg, unsigned nder, hipStream_t s, const AvgArgs& a, const DerArgs& d) {
+  hipLaunchKernelGGL((k_average_down<LAT, ST>), dim3(navg + nder), dim3(256), 0, s, a, navg, d);
 }
 
 static void pick_amr(int lat, int st, CfFn& cf, AvgFn& av, CfMoveFn& cm) {
@@ -126,10 +126,11 @@ constexpr int kMaxLev = 3;
 // stream-collide (k_step_cf).  us per coarse step of a cylinder with one
 // refined box, fills apart and taken along, by level-0 cells: 512x256 FP64
 // 75 and 63, FP32 65 and 56, FP16-shifted 66 and 55; 1448x724 104 and 96, 81
-// and 76, 76 and 73; beyond, the registers of the fill cost the step more
-// waves than the launch is worth: 2048x1024 FP32 96 and 98, FP16-shifted 83
-// and 89.
-constexpr int64_t kRideCells = (int64_t)1 << 20;
+// and 76, 76 and 73; beyond, the registers of the fill cost a step of
+// reduced storage more waves than the launch is worth: 2048x1024 FP32 96 and
+// 98, FP16-shifted 83 and 89, but FP64 131 and 121, 3000x1500 206 and 196,
+// 4096x2048 302 and 300.
+constexpr int64_t kRideCells = (int64_t)1 << 20, kRideCellsF64 = (int64_t)5 << 20;
 
 struct Amr {
   hipStream_t stream = nullptr;
@@ -141,7 +142,7 @@ struct Amr {
   double* dpartial[kMaxLev] = {nullptr, nullptr, nullptr};
   int64_t dblocks[kMaxLev] = {0, 0, 0};
   bool exported[kMaxLev] = {false, false, false};
-  int64_t ride_cells = kRideCells;   // ILBM_AMR_RIDE_CELLS
+  int64_t ride_cells = -1;   // ILBM_AMR_RIDE_CELLS; < 0: by storage
   bool cf_ready[kMaxLev] = {false, false, false};   // the next sub-step's fill (and kinematics) went with an earlier launch
   CfFn cffn = nullptr;
   CfMoveFn cfmovefn = nullptr;
@@ -319,9 +320,9 @@ struct Amr {
     regrid_on = true;
   }
 
-  void derived(int l, int sel) {
-    Level& V = *L[l];
-    if (!V.window) return;
+  // the derived fields of window slot sel, and the blocks of their launch
+  DerArgs der_args(int l, int sel, unsigned& nblk) const {
+    const Level& V = *L[l];
     DerArgs a{};
     a.M = V.Mw[sel];
     a.D = V.Dw[sel];
@@ -330,7 +331,14 @@ struct Amr {
     a.dim = dim;
     a.dx = V.c.dx[0]; a.dy = V.c.dx[1]; a.dz = V.c.dx[2];
     const int64_t nint = (int64_t)(a.n[0] - 2) * (a.n[1] - 2) * ((dim == 3) ? a.n[2] - 2 : 1);
-    if (nint > 0) hipLaunchKernelGGL(k_derived, dim3((unsigned)((nint + 255) / 256)), dim3(256), 0, stream, a);
+    nblk = nint > 0 ? (unsigned)((nint + 255) / 256) : 0;
+    return a;
+  }
+  void derived(int l, int sel) {
+    if (!L[l]->window) return;
+    unsigned nblk = 0;
+    const DerArgs a = der_args(l, sel, nblk);
+    if (nblk) hipLaunchKernelGGL(k_derived, dim3(nblk), dim3(256), 0, stream, a);
   }
 
   // GetDataMacro of level lc at `time` (AmrCoreLBM.cpp:2239-2269)
@@ -392,7 +400,8 @@ struct Amr {
   // apart.
   bool ride_args(int l, double time, bool first, CfRide& r) {
     Level& V = *L[l];
-    if (!pick_step_cf(V.lat, V.st, V.am) || V.ncells > ride_cells) return false;
+    const int64_t most = (ride_cells >= 0) ? ride_cells : (V.st == 0) ? kRideCellsF64 : kRideCells;
+    if (!pick_step_cf(V.lat, V.st, V.am) || V.ncells > most) return false;
     const unsigned nt = V.block.x * V.block.y;
     r = CfRide{};
     auto add = [&](int k, int m, double t, int buf) {
@@ -415,6 +424,7 @@ struct Amr {
     return r.n[0] + r.n[1] > 0;
   }
 
+  // with the derived fields of the window it completes
   void average_down(int l) {
     Level& C = *L[l];
     Level& F = *L[l + 1];
@@ -441,7 +451,9 @@ struct Amr {
     const StepArgs sa = C.step_args(false);
     for (int d = 0; d < 3; ++d) a.Fcol[d] = sa.Fcol[d];
     a.dpartial = dpartial[l];
-    avgfn(dim3((unsigned)dblocks[l]), stream, a);
+    unsigned nder = 0;
+    const DerArgs d = der_args(l, C.wsel, nder);
+    avgfn((unsigned)dblocks[l], nder, stream, a, d);
     // the covered cells keep 3 coarse cells inside the coarse box
     // (nest_geometry), so no boundary cell of level 0 is averaged down and
     // the slabs its stream-collide kernel wrote stay current
@@ -808,7 +820,6 @@ struct Amr {
       for (int i = 1; i <= 2; ++i)
         substep(l + 1, time + (double)(i - 1) * L[l + 1]->dt, last_chain && i == 2, row, i == 2, i == 1);
       average_down(l);
-      derived(l, V.wsel);
     }
     if (pre) patch_derived(l, V.t_new, Dfull[l][V.istep & 1]);
     HIPCHK(hipGetLastError());
