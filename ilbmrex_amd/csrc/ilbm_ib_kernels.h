@@ -596,7 +596,9 @@ __global__ void k_ib_entry_weights(IbArgs a, int64_t nent) {
 // serial scatter's order.
 __device__ inline void spread_cell_sum(const IbArgs& a, int64_t b, double tot[3]) {
   // kB entries per round: their list and marker-force loads are in flight
-  // together; the products are added in list order
+  // together; the products are added in list order.  (16 a round: 29 us
+  // against 15 for the lists of a 7-cell sphere in 3D, whose 10 to 30 entries
+  // leave most of a longer round's selects idle.)
   constexpr int kB = 8;
   const int nm = a.nm;
   const int e0 = a.rowptr[b], e1 = a.rowptr[b + 1];
@@ -869,6 +871,49 @@ __device__ __forceinline__ void correct_body(const IbArgs& a, int64_t b) {
 
 __global__ void k_ib_correct(IbArgs a) { correct_body(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x); }
 
+// One iteration of a fixed body after its marker forces, in one launch:
+// block 0 the marker sums, the next blocks spread to the non-empty band
+// cells and correct their velocities, and in the first iteration (it == 0)
+// further blocks start the other cells' EulerVel and EulerForceTotal.  That
+// first iteration interpolates from the macros and its correction starts
+// EulerVel from them, so no pass copies them first.  A single-iteration body
+// (ev_from_macro) only spreads, into EulerForceIter.  Additions as in
+// k_ib_begin, k_ib_spread_t, k_ib_sums and k_ib_correct, which run one after
+// the other where the stencils move.
+__global__ void __launch_bounds__(kSumsBlock) k_ib_spread_correct(IbArgs a, int it) {
+  if (blockIdx.x == 0) {
+    sums_body(a, a.F, it == 0);
+    return;
+  }
+  const int64_t bc = a.band_cells;
+  const int nl = (a.n_ne + kSumsBlock - 1) / kSumsBlock;
+  const int blk = (int)blockIdx.x - 1;
+  int64_t b;
+  double tot[3] = {0.0, 0.0, 0.0};
+  if (blk < nl) {
+    const int ci = blk * kSumsBlock + (int)threadIdx.x;
+    if (ci >= a.n_ne) return;
+    b = a.ne_cells[ci];
+    spread_cell_sum(a, b, tot);
+  } else {
+    b = (int64_t)(blk - nl) * kSumsBlock + threadIdx.x;
+    if (b >= bc || a.rowptr[b] != a.rowptr[b + 1]) return;
+  }
+  for (int c = 0; c < 3; ++c) {
+    const int64_t o = c * bc + b;
+    if (a.ev_from_macro) {
+      a.EFI[o] = tot[c];
+    } else if (it == 0) {
+      const double m = (c == 2 && a.dim != 3) ? 0.0 : a.Mband[(c + 1) * bc + b];
+      a.EV[o] = m + a.dt * tot[c];
+      a.EFT[o] = 0.0 + tot[c];
+    } else {
+      a.EV[o] += a.dt * tot[c];
+      a.EFT[o] += tot[c];
+    }
+  }
+}
+
 __global__ void k_ib_export(IbArgs a) {
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= a.band_cells) return;
@@ -1109,7 +1154,7 @@ __device__ __forceinline__ void export_fixup_body(const IbArgs& a, const GridGeo
     b = t.b;
     active = t.active;
   }
-  if (active && (kPre || kGather)) {
+  if (active && (kPre || kGather || MODE == 5)) {
     for (int c = 0; c < 4; ++c) mac[c] = a.Mband[c * a.band_cells + b];
     if constexpr (kPre) {
       const int bi = (int)(b % a.band_n[0]);
@@ -1121,7 +1166,7 @@ __device__ __forceinline__ void export_fixup_body(const IbArgs& a, const GridGeo
   }
   if constexpr (kGather) gather_tile_sum<LAT::D == 3, MODE == 4>(a, gather_tile_of<MODE == 4>(a, blk), cell_tot);
   if (active) {
-    if constexpr (!(kPre || kGather)) mac[0] = a.Mband[b];
+    if constexpr (!(kPre || kGather || MODE == 5)) mac[0] = a.Mband[b];
     const double rho = mac[0];
     if constexpr (MODE == 0) {
       const double* tot = a.ev_from_macro ? a.EFI : a.EFT;
@@ -1130,6 +1175,13 @@ __device__ __forceinline__ void export_fixup_body(const IbArgs& a, const GridGeo
       cell_tot[2] = tot[2 * a.band_cells + b];
     } else if constexpr (MODE == 1) {
       spread_cell_sum(a, b, cell_tot);
+    } else if constexpr (MODE == 5) {
+      // the last of several iterations, on the sum of those before it
+      const double t0 = a.EFT[b], t1 = a.EFT[a.band_cells + b], t2 = a.EFT[2 * a.band_cells + b];
+      spread_cell_sum(a, b, cell_tot);
+      cell_tot[0] = t0 + cell_tot[0];
+      cell_tot[1] = t1 + cell_tot[1];
+      cell_tot[2] = t2 + cell_tot[2];
     }
     fx = a.dt * rho * cell_tot[0];
     fy = a.dt * rho * cell_tot[1];
@@ -1139,12 +1191,12 @@ __device__ __forceinline__ void export_fixup_body(const IbArgs& a, const GridGeo
     a.Fband[2 * a.band_cells + b] = fz;
     if (!(fx == 0.0 && fy == 0.0 && fz == 0.0)) {
       if constexpr (!kPre) {
-        const int bi = (int)(b % a.band_n[0]);
-        const int bj = (int)((b / a.band_n[0]) % a.band_n[1]);
-        const int bk = (int)(b / ((int64_t)a.band_n[0] * a.band_n[1]));
-        self = g.idx(a.band_lo[0] + bi, a.band_lo[1] + bj, a.band_lo[2] + bk);
+        // (a band's rows fit 32 bits)
+        const uint32_t row = (uint32_t)(b / a.band_n[0]), bi = (uint32_t)(b - (int64_t)row * a.band_n[0]);
+        const uint32_t bk = row / (uint32_t)a.band_n[1], bj = row - bk * (uint32_t)a.band_n[1];
+        self = g.idx(a.band_lo[0] + (int)bi, a.band_lo[1] + (int)bj, a.band_lo[2] + (int)bk);
       }
-      if constexpr (!(kPre || kGather))
+      if constexpr (!(kPre || kGather || MODE == 5))
         for (int c = 1; c < 4; ++c) mac[c] = a.Mband[c * a.band_cells + b];
       const T ux = T(mac[1]), uy = T(mac[2]), uz = T(mac[3]);
       const T fac = T(1.0) - T(0.5) / T(tau);
@@ -1434,11 +1486,11 @@ __device__ __forceinline__ void force_record_body(const IbArgs& a, const RecArgs
 
 __global__ void __launch_bounds__(256) k_force_record(IbArgs a, RecArgs rec, int nblk) { force_record_body(a, rec, nblk); }
 
-// Single-iteration forcing: the marker sums (k_ib_sums, same tree) and the
-// record in one launch.
+// The marker sums (k_ib_sums, same tree) of the only or last iteration and
+// the record in one launch.
 __device__ __forceinline__ void sums_record_body(const IbArgs& a, const RecArgs& rec, int nblk) {
   __shared__ double lds[3][16];
-  sums_body(a, a.F, 1);
+  sums_body(a, a.F, a.nloop == 1);
   __syncthreads();
   const int tid = lin_tid(), nt = lin_nt();
   double acc[3] = {0.0, 0.0, 0.0};

@@ -429,7 +429,8 @@ static void launch_init(dim3 g, dim3 b, hipStream_t s, const InitArgs& a) {
 // mode 0: export of EulerForceIter / Total; 1: fused CSR spreading (thread
 // per band cell); 2: fused gather spreading of a moving body (marker order);
 // 3: fused CSR spreading, one wavefront per non-empty band cell; 4: as 2 in
-// tree order (16 x 4 tiles, four wavefronts per tile)
+// tree order (16 x 4 tiles, four wavefronts per tile); 5: as 1 for the last
+// of several iterations
 template <class LAT, class ST>
 static void launch_fix(int mode, dim3 g, dim3 b, hipStream_t s, const IbArgs& a, const GridGeom& gg, void* buf,
                        double tau, const RecArgs& r) {
@@ -437,6 +438,7 @@ static void launch_fix(int mode, dim3 g, dim3 b, hipStream_t s, const IbArgs& a,
   else if (mode == 1) hipLaunchKernelGGL((k_ib_export_fixup<LAT, ST, 1>), g, b, 0, s, a, gg, buf, tau, r);
   else if (mode == 2) hipLaunchKernelGGL((k_ib_export_fixup<LAT, ST, 2>), g, b, 0, s, a, gg, buf, tau, r);
   else if (mode == 4) hipLaunchKernelGGL((k_ib_export_fixup<LAT, ST, 4>), g, b, 0, s, a, gg, buf, tau, r);
+  else if (mode == 5) hipLaunchKernelGGL((k_ib_export_fixup<LAT, ST, 5>), g, b, 0, s, a, gg, buf, tau, r);
   else hipLaunchKernelGGL((k_ib_export_fixup<LAT, ST, 0>), g, b, 0, s, a, gg, buf, tau, r);
 }
 template <class LAT, class ST>
@@ -657,6 +659,7 @@ struct Level {
   // the same step or, with no slab launch, as the last block of the
   // stream-collide launch
   bool rec_to_ghost = false, rec_held = false;
+  const bool ib_fused = !(std::getenv("ILBM_IB_FUSED") && std::getenv("ILBM_IB_FUSED")[0] == '0');
   // k_step writes the x-face ghost slabs of the next step (ghost_write);
   // slabs_fresh: the current buffer's slabs were written by the last step
   // (or restored with it); a gfuse level's boundary layer is then stale
@@ -1537,10 +1540,29 @@ struct Level {
     return a;
   }
 
+  // Several iterations of a body with fixed lists: sums and correction with
+  // the spreading, the last spreading with the export, the last sums with
+  // the record (k_ib_spread_correct): 5 or 6 launches per step in place of 13
+  // with two iterations, sphere 141x34x106 FP64 125 -> 105 us (with the
+  // interpolation's 2 x 4.5).  ILBM_IB_FUSED=0: separate launches.
+  bool fuse_iter() const {
+    const int nloop = (c.coupling_method == 1) ? 1 : std::max(c.loop_ns, 1);
+    return nloop > 1 && !moving && n_ne > 0 && ib_fused;
+  }
+  void launch_interp(IbArgs a, bool from_macro) {
+    if (from_macro) a.ev_from_macro = 1;
+    hipLaunchKernelGGL(k_ib_interp, dim3(interp_blocks(nm, a.tree != 0, c.dim)), dim3(64 * kInterpWaves), 0, stream, a);
+  }
+  void spread_correct(const IbArgs& a, int it) {
+    const unsigned nl = (unsigned)((n_ne + kSumsBlock - 1) / kSumsBlock);
+    const unsigned nb = (it == 0) ? (unsigned)((band_cells + kSumsBlock - 1) / kSumsBlock) : 0;
+    hipLaunchKernelGGL(k_ib_spread_correct, dim3(1 + nl + (a.ev_from_macro ? 0 : nb)), dim3(kSumsBlock), 0, stream, a, it);
+  }
+
   // how the IB force is exported (see launch_fix) and its block count
   int fix_mode() const {
     const int nloop = (c.coupling_method == 1) ? 1 : std::max(c.loop_ns, 1);
-    if (nloop > 1) return 0;
+    if (nloop > 1) return fuse_iter() ? 5 : 0;
     if (dev_kin) return ib_tree ? 4 : 2;
     return (c.dim == 3 && spread_wave) ? 3 : 1;
   }
@@ -1615,17 +1637,21 @@ struct Level {
     const unsigned gb = (unsigned)((band_cells + tb - 1) / tb);
     const bool use_ivc = a.use_ivc != 0;
     const int nloop = a.nloop;
-    if (!a.ev_from_macro) hipLaunchKernelGGL(k_ib_begin, dim3(gb), dim3(tb), 0, stream, a);
+    const bool fused = fuse_iter();
+    if (!a.ev_from_macro && !fused) hipLaunchKernelGGL(k_ib_begin, dim3(gb), dim3(tb), 0, stream, a);
     for (int it = 0; it < nloop; ++it) {
       a.first_iter = (it == 0) ? 1 : 0;
-      hipLaunchKernelGGL(k_ib_interp, dim3(interp_blocks(nm, a.tree != 0, c.dim)), dim3(64 * kInterpWaves), 0,
-                         stream, a);
+      launch_interp(a, fused && it == 0);
       if (ib_mark == 1 && nloop == 1 && !use_ivc) ib_sig = xsignal(stream, X_IB);
       if (use_ivc) {
         hipLaunchKernelGGL(k_ib_ivc_rhs, dim3((nm + tb - 1) / tb), dim3(tb), 0, stream, a);
         hipLaunchKernelGGL(k_ib_ivc_matvec, dim3((nm + 3) / 4), dim3(256), 0, stream, a);
       }
       if (nloop == 1) break;  // single iteration: spreading fused into the export
+      if (fused) {
+        if (it < nloop - 1) spread_correct(a, it);   // the last one's: with the export and the record
+        continue;
+      }
       if (dev_kin)
         hipLaunchKernelGGL(k_ib_spread_all, dim3(gb), dim3(tb), 0, stream, a);
       else if (n_ne)
@@ -1652,6 +1678,12 @@ struct Level {
       } else if (rec_enable) {
         hipLaunchKernelGGL(k_sums_record, dim3(1), dim3(kSumsBlock), 0, stream, a, r, (int)gfix);
       }
+    } else if (rec_enable && fused && rec_to_ghost && block.x * block.y == (unsigned)kSumsBlock) {
+      rec_held = true;
+      held_a = a; held_r = r; held_nblk = (int)gfix;
+    } else if (rec_enable && fused) {
+      // (on the forcing's stream: the next step's first iteration restarts the sums)
+      hipLaunchKernelGGL(k_sums_record, dim3(1), dim3(kSumsBlock), 0, stream, a, r, (int)gfix);
     } else if (rec_enable) {
       hipLaunchKernelGGL(k_force_record, dim3(1), dim3(256), 0, stream, a, r, (int)gfix);
     }
@@ -1674,14 +1706,18 @@ struct Level {
     IbArgs a = ib_args();
     const int tb = 256;
     const unsigned gb = (unsigned)((band_cells + tb - 1) / tb);
-    if (!a.ev_from_macro) hipLaunchKernelGGL(k_ib_begin, dim3(gb), dim3(tb), 0, stream, a);
+    const bool fused = !moving && n_ne > 0 && ib_fused;
+    if (!a.ev_from_macro && !fused) hipLaunchKernelGGL(k_ib_begin, dim3(gb), dim3(tb), 0, stream, a);
     for (int it = 0; it < a.nloop; ++it) {
       a.first_iter = (it == 0) ? 1 : 0;
-      hipLaunchKernelGGL(k_ib_interp, dim3(interp_blocks(nm, a.tree != 0, c.dim)), dim3(64 * kInterpWaves), 0,
-                         stream, a);
+      launch_interp(a, fused && it == 0);
       if (a.use_ivc) {
         hipLaunchKernelGGL(k_ib_ivc_rhs, dim3((nm + tb - 1) / tb), dim3(tb), 0, stream, a);
         hipLaunchKernelGGL(k_ib_ivc_matvec, dim3((nm + 3) / 4), dim3(256), 0, stream, a);
+      }
+      if (fused) {
+        spread_correct(a, it);
+        continue;
       }
       if (dev_kin)
         hipLaunchKernelGGL(k_ib_spread_all, dim3(gb), dim3(tb), 0, stream, a);
