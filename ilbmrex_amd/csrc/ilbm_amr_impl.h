@@ -12,7 +12,8 @@
 //                exports the window macros), derived fields every
 //                regrid_int steps, then twice substep(1) and
 //                AverageDownTo(0) + derived fields
-//   substep(l):  ghost slabs from level l-1 at the substep's time, IB
+//   substep(l):  ghost slabs from level l-1 at the substep's time (in 2D
+//                mostly filled by an earlier step's launch, k_step_cf), IB
 //                forcing (finest), stream-collide (exports f and macros on
 //                the second substep for the average-down), recursion
 //   Sum(Rho) of level 0 and the finest level's force record (Evolve,

@@ -14,6 +14,11 @@
 //   k_ib_correct   EulerVel += dt * Iter, Total += Iter             (:1514-1520, :1878-1879)
 //   k_ib_export    F = dt * rho * Total                             (:1889-1912)
 //
+// Fused forms: k_ib_spread_correct (spread, sums and correct of a fixed body),
+// k_ib_export_fixup (export with the Guo term, and with the last spreading),
+// k_sums_record, and for fixed 2D bodies the whole forcing in body tiles
+// (k_step_body).
+//
 // Spreading is a deterministic gather: every band cell walks a precomputed
 // list of (marker, stencil point) contributions in marker order, so the
 // per-cell sums are evaluated in the same order as the reference's serial

@@ -1,7 +1,7 @@
 // Resident MI355X IB-LBM level: host driver (the AdvancePhiAtLevel /
 // Evolve / IBMarkerDF roles of the reference) and the C ABI of include/ilbm.h.
 //
-// Per coarse step, all on one stream, no host synchronisation:
+// Per coarse step, without host synchronisation:
 //   [IB]   k_ib_*             F^{n+1} on the band from macro^n (IBMarkerDF::update_forcing)
 //   [IB]   k_ib_export_fixup  export F, Guo term of step n+1 on band cells
 //                             (collide_forced.H:22-50), force.dat row
@@ -9,6 +9,9 @@
 //   [wall] k_fill_ghosts      ghost slabs (FillPatch / bounce-back)
 //          k_step             pull + macros + BGK (AdvanceLBMAtLevel.cpp:223-386)
 //                             and Sum(Rho) (AmrCoreLBM.cpp:378)
+// A fixed 2D body's step is one launch, k_step_body, with the forcing of the
+// next step in body tiles (advance_body); large IB levels run the forcing
+// beside the cells far from it on further streams (split_step3).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
