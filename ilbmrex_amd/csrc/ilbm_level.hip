@@ -16,7 +16,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -25,23 +24,13 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "ilbm.h"
+#include "ilbm_host_copy.h"
 #include "ilbm_ib_kernels.h"
 
 namespace ilbm {
-
-struct HipError {
-  hipError_t e;
-};
-#define HIPCHK(x)                                   \
-  do {                                              \
-    hipError_t e_ = (x);                            \
-    if (e_ != hipSuccess) throw ::ilbm::HipError{e_}; \
-  } while (0)
 
 struct StatusError {
   int status;
@@ -66,85 +55,6 @@ static void dev_free(void* p) {
 }
 
 static constexpr double kPi = 3.14159265358979323846;
-
-// Device-to-host copies of whole fields into a caller's ordinary memory.
-// hipMemcpy stages such a copy through one buffer and one core, and the
-// destination is usually fresh memory whose pages the copy touches first
-// (134 MB of macros: 14 ms, 10 GB/s).  Here up to kWorkers threads each own a
-// pinned buffer: a thread queues the transfer of its next slice, waits for it
-// and copies it out, so that transfers run behind each other while the cores
-// share the page faults and the copying: 134 MB in 3.3 ms, 537 MB 51 -> 11.8
-// ms (45 GB/s).  The buffers live with the level (allocated by its first
-// large copy in 2.3 ms, given back with it); copies below kDirect bytes
-// (1.8 ms plain), and any for which no thread can be had, are plain.
-struct HostCopy {
-  static constexpr int kWorkers = 8;
-  static constexpr size_t kSlice = (size_t)4 << 20;
-  static constexpr size_t kDirect = (size_t)32 << 20;
-  char* pinned = nullptr;
-  hipEvent_t ev[kWorkers] = {};
-
-  HostCopy() = default;
-  HostCopy(const HostCopy&) = delete;
-  HostCopy& operator=(const HostCopy&) = delete;
-  ~HostCopy() {
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (pinned) (void)hipHostFree(pinned);
-  }
-
-  // ordered behind the work of stream s; returns when dst is complete
-  void copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes < kDirect || !ready()) {
-      HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-      HIPCHK(hipStreamSynchronize(s));
-      return;
-    }
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
-    const size_t slices = (bytes + kSlice - 1) / kSlice;
-    std::atomic<size_t> next{0};
-    std::atomic<int> failed{(int)hipSuccess};
-    auto work = [&](int w) {
-      hipError_t e = hipSetDevice(dev);
-      char* buf = pinned + (size_t)w * kSlice;
-      while (e == hipSuccess) {
-        const size_t i = next.fetch_add(1);
-        if (i >= slices) return;
-        const size_t off = i * kSlice, n = std::min(kSlice, bytes - off);
-        e = hipMemcpyAsync(buf, static_cast<const char*>(src) + off, n, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(ev[w], s);
-        if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
-        if (e == hipSuccess) std::memcpy(static_cast<char*>(dst) + off, buf, n);
-      }
-      failed = (int)e;
-    };
-    std::thread th[kWorkers];
-    const int want = (int)std::min<size_t>(kWorkers, slices);
-    for (int w = 1; w < want; ++w) {
-      try {
-        th[w] = std::thread(work, w);
-      } catch (const std::system_error&) {
-        break;   // the threads there are take every slice
-      }
-    }
-    work(0);
-    for (std::thread& t : th)
-      if (t.joinable()) t.join();
-    HIPCHK((hipError_t)failed.load());
-  }
-
- private:
-  bool ready() {
-    if (pinned) return true;
-    for (hipEvent_t& e : ev)
-      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-    void* p = nullptr;
-    if (hipHostMalloc(&p, kWorkers * kSlice, hipHostMallocDefault) != hipSuccess) return false;
-    pinned = static_cast<char*>(p);
-    return true;
-  }
-};
 
 // ---------------------------------------------------------------------------
 // Marker geometry on the host (IBMarkerDF::build_markers,
