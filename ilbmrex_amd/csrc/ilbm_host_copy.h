@@ -32,7 +32,8 @@ struct HipError {
 // ms (45 GB/s).  The buffers live with the level (allocated by its first
 // large copy in 2.3 ms, given back with it).  Copies below kDirect bytes
 // (1.8 ms plain) are plain, and so is one that finds the buffers in use by
-// another thread's copy of the same level.
+// another thread's copy of the same level or cannot have them (the runtime's
+// last error, which the next launch check would report, is then cleared).
 struct HostCopy {
   static constexpr int kWorkers = 8;
   static constexpr size_t kSlice = (size_t)4 << 20;
@@ -95,12 +96,14 @@ struct HostCopy {
  private:
   bool ready() {
     if (pinned) return true;
+    bool ok = true;
     for (hipEvent_t& e : ev)
-      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+      ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
     void* p = nullptr;
-    if (hipHostMalloc(&p, kWorkers * kSlice, hipHostMallocDefault) != hipSuccess) return false;
-    pinned = static_cast<char*>(p);
-    return true;
+    ok = ok && hipHostMalloc(&p, kWorkers * kSlice, hipHostMallocDefault) == hipSuccess;
+    if (ok) pinned = static_cast<char*>(p);
+    else (void)hipGetLastError();
+    return ok;
   }
 };
 

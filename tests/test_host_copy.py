@@ -147,3 +147,7 @@ def test_one_copy(program):
 
 def test_two_threads_read_one_level(program):
     assert _run(program, "threads") == 0
+
+
+def test_no_pinned_memory_leaves_no_error_behind(program):
+    assert _run(program, "pinned") == 0
