@@ -51,21 +51,34 @@ struct HostCopy {
     if (pinned) (void)hipHostFree(pinned);
   }
 
+  // The device of stream s as the calling thread's, while the copy runs: its
+  // events must be of the stream's device, whichever is current.
+  struct OnDevice {
+    int dev = 0, prev = 0;
+    explicit OnDevice(hipStream_t s) {
+      HIPCHK(hipGetDevice(&prev));
+      HIPCHK(hipStreamGetDevice(s, &dev));
+      if (dev != prev) HIPCHK(hipSetDevice(dev));
+    }
+    ~OnDevice() {
+      if (dev != prev) (void)hipSetDevice(prev);
+    }
+  };
+
   // ordered behind the work of stream s; returns when dst is complete
   void copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    const OnDevice on(s);
     std::unique_lock<std::mutex> lock(busy, std::defer_lock);
     if (bytes < kDirect || !lock.try_lock() || !ready()) {
       HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
       HIPCHK(hipStreamSynchronize(s));
       return;
     }
-    int dev = 0;
-    HIPCHK(hipGetDevice(&dev));
     const size_t slices = (bytes + kSlice - 1) / kSlice;
     std::atomic<size_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     auto work = [&](int w) {
-      hipError_t e = hipSetDevice(dev);
+      hipError_t e = hipSetDevice(on.dev);
       char* buf = pinned + (size_t)w * kSlice;
       while (e == hipSuccess) {
         const size_t i = next.fetch_add(1);

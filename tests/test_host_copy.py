@@ -151,3 +151,7 @@ def test_two_threads_read_one_level(program):
 
 def test_no_pinned_memory_leaves_no_error_behind(program):
     assert _run(program, "pinned") == 0
+
+
+def test_level_of_another_device_than_the_current_one(program):
+    assert _run(program, "device") == 0
