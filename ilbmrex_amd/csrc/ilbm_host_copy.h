@@ -7,8 +7,8 @@
 #include <atomic>
 #include <cstddef>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace ilbm {
@@ -96,8 +96,8 @@ struct HostCopy {
     for (int w = 1; w < want; ++w) {
       try {
         th[w] = std::thread(work, w);
-      } catch (const std::system_error&) {
-        break;   // the threads there are take every slice
+      } catch (const std::exception&) {   // no thread, or no memory for one
+        break;                             // the threads there are take every slice
       }
     }
     work(0);

@@ -155,3 +155,7 @@ def test_no_pinned_memory_leaves_no_error_behind(program):
 
 def test_level_of_another_device_than_the_current_one(program):
     assert _run(program, "device") == 0
+
+
+def test_no_host_memory_for_a_thread(program):
+    assert _run(program, "memory") == 0
