@@ -741,7 +741,7 @@ struct Level {
     dev_free(xm_d); dev_free(ut_d); dev_free(U_d); dev_free(F_d); dev_free(Mm_d);
     dev_free(base_d); dev_free(wts_d); dev_free(scale_d); dev_free(rhs_d); dev_free(sums_d);
     dev_free(Ainv_d); dev_free(rowptr_d); dev_free(entm_d); dev_free(entc_d); dev_free(entw_d); dev_free(frstate_d);
-    dev_free(body_mask); dev_free(body_int); dev_free(body_dbl); dev_free(body_tiles); dev_free(body_F); dev_free(body_Fband);
+    free_body();
     dev_free(ne_d); dev_free(nee_d); dev_free(fpartial); dev_free(clock_d); dev_free(xref_d); dev_free(chunk_d);
     for (int b = 0; b < 2; ++b) { dev_free(Mw[b]); dev_free(Dw[b]); }
     if (stream && own_stream) (void)hipStreamDestroy(stream);
@@ -1070,9 +1070,24 @@ struct Level {
   // separate forcing kernels).  A body they cannot hold -- stencils beyond
   // the ghost layers, lists over the LDS budget, more iterations than
   // kBodyLoops -- and large levels of reduced storage keep the separate
-  // kernels too.
+  // kernels too, and so does a level without memory left for the tables:
+  // advance never starts on part of them.
   void setup_body() {
     body_tried = true;
+    try {
+      build_body();
+    } catch (const StatusError& e) {
+      free_body();
+      if (e.status != ILBM_ERR_ALLOC) throw;
+      (void)hipGetLastError();   // nothing failed for the caller
+    }
+  }
+  void free_body() {
+    dev_free(body_mask); dev_free(body_int); dev_free(body_dbl); dev_free(body_tiles); dev_free(body_F); dev_free(body_Fband);
+    body_mask = nullptr; body_int = nullptr; body_dbl = nullptr; body_tiles = nullptr;
+    body_F = body_Fband = nullptr;
+  }
+  void build_body() {
     const char* e = std::getenv("ILBM_BODY_TILES");
     const int nloop = ib_args().nloop;
     if (c.dim != 2 || moving || cf || !stepbodyfn || n_ne == 0 || nloop > kBodyLoops || (e && e[0] == '0')) return;
@@ -1200,6 +1215,8 @@ struct Level {
     body_int = dev_alloc<int>(ints.size());
     body_dbl = dev_alloc<double>(em.size() + ghv.size());
     body_tiles = dev_alloc<BodyTile>(tiles.size());
+    body_F = dev_alloc<double>(3 * (size_t)nm * nloop);
+    body_Fband = dev_alloc<double>(3 * band_cells);
     HIPCHK(hipMemcpyAsync(body_mask, mask.data(), mask.size(), hipMemcpyHostToDevice, stream));
     HIPCHK(hipMemcpyAsync(body_int, ints.data(), sizeof(int) * ints.size(), hipMemcpyHostToDevice, stream));
     HIPCHK(hipMemcpyAsync(body_tiles, tiles.data(), sizeof(BodyTile) * tiles.size(), hipMemcpyHostToDevice, stream));
@@ -1235,10 +1252,6 @@ struct Level {
   // the next step's forcing in its first blocks.  Step s uses slot
   // (nsteps - 1 - s) & 1, so the last one leaves its force in slot 0.
   void advance_body(int nsteps, bool want_state) {
-    if (!body_F) {
-      body_F = dev_alloc<double>(3 * (size_t)nm * ib_args().nloop);
-      body_Fband = dev_alloc<double>(3 * band_cells);
-    }
     const int64_t npad = wrap ? 0 : slabs.face_off[slabs.nface];
     BodyArgs B[2] = {body_args(0), body_args(1)};
     const bool ivc = B[0].ib.use_ivc != 0;

@@ -1,0 +1,76 @@
+"""Device memory that runs out while an advance sets up what only its fast path
+needs: the advance takes the other path, or fails and can be called again,
+with the results of an undisturbed run.  A library loaded before the
+framework's in a process of its own refuses one allocation."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+REFUSE = r"""
+#include <dlfcn.h>
+#include <cstddef>
+static int left = 0;
+extern "C" void refuse(int k) { left = k; }           // the k-th allocation from now
+extern "C" int pending() { return left; }
+extern "C" int hipMalloc(void** p, size_t n) {
+  static auto real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), "hipMalloc");
+  if (left > 0 && --left == 0) return 2;              // hipErrorOutOfMemory
+  return real(p, n);
+}
+"""
+
+PROGRAM = """
+import ctypes, sys
+lib = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+from ilbmrex_amd import config as cf
+from ilbmrex_amd.native import Level
+
+def results(case, first, last, must_succeed):
+    # an advance for each allocation refused, first to last
+    init = cf.uniform_init(case, u=(case.U0, 0.0, 0.0))
+    with Level(case, init) as lev:
+        lev.advance(1)
+        lev.advance(8, want_state=True)
+        ref = lev.f(), lev.force_history()
+    for k in range(first, last + 1):
+        print("refusing allocation", k, "of the first advance", flush=True)
+        with Level(case, init) as lev:
+            lib.refuse(k)
+            try:
+                lev.advance(1)
+            except RuntimeError:
+                assert not must_succeed, k
+                lev.advance(1)
+            assert lib.pending() == 0, "the advance allocates less than that"
+            lev.advance(8, want_state=True)
+            got = lev.f(), lev.force_history()
+        assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1]), k
+"""
+
+
+def _child(tmp_path, body, **env):
+    (tmp_path / "refuse.cpp").write_text(REFUSE)
+    (tmp_path / "program.py").write_text(PROGRAM + body)
+    lib = str(tmp_path / "librefuse.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", lib, str(tmp_path / "refuse.cpp"), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-u", str(tmp_path / "program.py"), lib], cwd=ROOT, timeout=100,
+                       env={**os.environ, "PYTHONPATH": ROOT, **env}, capture_output=True, text=True)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0
+
+
+def test_body_tiles_without_memory_for_their_tables(tmp_path):
+    # the first six allocations of the advance are the tiles'; the seventh,
+    # the Sum(Rho) ring, may fail it
+    _child(tmp_path, """
+case = cf.cylinder_2d(nx=96, ny=64, D=16.0, xc=32.0, yc=32.0)
+results(case, 1, 6, True)
+results(case, 7, 7, False)
+""")
