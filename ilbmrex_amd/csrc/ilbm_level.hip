@@ -37,18 +37,20 @@ struct StatusError {
   std::string msg;
 };
 
-template <class T>
-static T* dev_alloc(size_t count) {
-  if (count == 0) count = 1;
-  void* p = nullptr;
-  if (hipMalloc(&p, count * sizeof(T)) != hipSuccess) throw StatusError{ILBM_ERR_ALLOC, "hipMalloc"};
-  return static_cast<T*>(p);
-}
+// (a refused allocation is thrown here; the next launch check must not report
+// it again from the runtime's last error)
 static void* dev_alloc_bytes(size_t bytes) {
   void* p = nullptr;
   if (bytes == 0) bytes = 1;
-  if (hipMalloc(&p, bytes) != hipSuccess) throw StatusError{ILBM_ERR_ALLOC, "hipMalloc"};
+  if (hipMalloc(&p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    throw StatusError{ILBM_ERR_ALLOC, "hipMalloc"};
+  }
   return p;
+}
+template <class T>
+static T* dev_alloc(size_t count) {
+  return static_cast<T*>(dev_alloc_bytes(std::max<size_t>(count, 1) * sizeof(T)));
 }
 static void dev_free(void* p) {
   if (p) (void)hipFree(p);
@@ -1079,7 +1081,6 @@ struct Level {
     } catch (const StatusError& e) {
       free_body();
       if (e.status != ILBM_ERR_ALLOC) throw;
-      (void)hipGetLastError();   // nothing failed for the caller
     }
   }
   void free_body() {
@@ -1913,24 +1914,32 @@ struct Level {
       nblocks_ring = (int64_t)grid_ring.x * grid_ring.y * grid_ring.z;
       const char* two = std::getenv("ILBM_OVERLAP_TWO_REGIONS");
       if (two && two[0] == '1') ring_ok = false;
-      HIPCHK(hipStreamCreateWithFlags(&stream_b, hipStreamNonBlocking));
-      for (hipEvent_t* e : {&ev_a, &ev_b})
-        HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
-      if (ring_ok && ring_stream == RING_OWN) {
-        HIPCHK(hipStreamCreateWithFlags(&stream_d, hipStreamNonBlocking));
-        HIPCHK(hipEventCreateWithFlags(&ev_d, hipEventDisableTiming));
-      }
-      for (hipEvent_t& e : xev) HIPCHK(hipEventCreateWithFlags(&e, step_event_flags()));
+      // what an earlier call left here when it failed is kept; stream_b, made
+      // last, says that everything is there
+      auto make_event = [](hipEvent_t& e, unsigned flags) {
+        if (!e) HIPCHK(hipEventCreateWithFlags(&e, flags));
+      };
+      auto make_stream = [](hipStream_t& st) {
+        if (!st) HIPCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+      };
+      make_event(ev_a, hipEventDisableTiming);
+      make_event(ev_b, hipEventDisableTiming);
+      for (hipEvent_t& e : xev) make_event(e, step_event_flags());
       if (async_record()) {
-        HIPCHK(hipStreamCreateWithFlags(&stream_c, hipStreamNonBlocking));
-        HIPCHK(hipEventCreateWithFlags(&ev_c, hipEventDisableTiming));
         F_ring[0] = F_d;
         fp_ring[0] = fpartial;
-        for (int k = 0; k < kRecRing; ++k) {
-          if (k > 0 && !F_ring[k]) F_ring[k] = dev_alloc<double>(3 * nm);
-          if (k > 0 && !fp_ring[k]) fp_ring[k] = dev_alloc<double>(fpartial_n);
+        for (int k = 1; k < kRecRing; ++k) {
+          if (!F_ring[k]) F_ring[k] = dev_alloc<double>(3 * nm);
+          if (!fp_ring[k]) fp_ring[k] = dev_alloc<double>(fpartial_n);
         }
+        make_event(ev_c, hipEventDisableTiming);
+        make_stream(stream_c);
       }
+      if (ring_ok && ring_stream == RING_OWN) {
+        make_event(ev_d, hipEventDisableTiming);
+        make_stream(stream_d);
+      }
+      make_stream(stream_b);
     }
     return true;
   }

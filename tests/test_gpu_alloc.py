@@ -20,8 +20,7 @@ extern "C" void refuse(int k) { left = k; }           // the k-th allocation fro
 extern "C" int pending() { return left; }
 extern "C" int hipMalloc(void** p, size_t n) {
   static auto real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), "hipMalloc");
-  if (left > 0 && --left == 0) return 2;              // hipErrorOutOfMemory
-  return real(p, n);
+  return real(p, left > 0 && --left == 0 ? (size_t)1 << 60 : n);   // more than there is
 }
 """
 
@@ -74,3 +73,11 @@ case = cf.cylinder_2d(nx=96, ny=64, D=16.0, xc=32.0, yc=32.0)
 results(case, 1, 6, True)
 results(case, 7, 7, False)
 """)
+
+
+def test_overlapped_step_without_memory_for_its_record_slots(tmp_path):
+    # six slots of the record, then the Sum(Rho) rings of the three regions
+    _child(tmp_path, """
+case = cf.sphere_3d(nx=128, ny=96, nz=96, D=10.0, center=(48.0, 47.6, 48.3), storage=cf.STORE_F32)
+results(case, 1, 9, False)
+""", ILBM_OVERLAP_BYTES="0")
