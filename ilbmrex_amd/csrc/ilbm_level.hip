@@ -1004,7 +1004,7 @@ struct Level {
     xm_d = dev_alloc<double>(3 * nm);
     ut_d = dev_alloc<double>(3 * nm);
     U_d = dev_alloc<double>(3 * nm);
-    F_d = dev_alloc<double>(3 * (size_t)nm * std::max(c.loop_ns, 1));   // body tiles keep every iteration's
+    F_d = dev_alloc<double>(3 * nm);
     Mm_d = dev_alloc<double>(3 * nm);
     base_d = dev_alloc<int>(3 * nm);
     wts_d = dev_alloc<double>(15 * nm);
@@ -1228,6 +1228,14 @@ struct Level {
     hipLaunchKernelGGL(k_gather_doubles, dim3((unsigned)((em.size() + 255) / 256)), dim3(256), 0, stream,
                        (const double*)entw_d, (const int*)(body_int + osrc), body_dbl, (int64_t)em.size());
     HIPCHK(hipGetLastError());
+    if (nloop > 1) {   // the tiles keep every iteration's marker forces, the last one's first
+      double* F = dev_alloc<double>(3 * (size_t)nm * nloop);
+      std::swap(F, F_d);
+      const hipError_t e = hipMemcpyAsync(F_d, F, sizeof(double) * 3 * nm, hipMemcpyDeviceToDevice, stream);
+      (void)hipStreamSynchronize(stream);
+      dev_free(F);
+      HIPCHK(e);
+    }
     HIPCHK(hipStreamSynchronize(stream));   // host vectors go out of scope
     body.tiles = body_tiles;
     body.ntile = (int)tiles.size();

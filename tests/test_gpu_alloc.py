@@ -72,6 +72,7 @@ def test_body_tiles_without_memory_for_their_tables(tmp_path):
 case = cf.cylinder_2d(nx=96, ny=64, D=16.0, xc=32.0, yc=32.0)
 results(case, 1, 6, True)
 results(case, 7, 7, False)
+results(case.replace(loop_ns=2), 1, 7, True)
 """)
 
 
@@ -81,3 +82,18 @@ def test_overlapped_step_without_memory_for_its_record_slots(tmp_path):
 case = cf.sphere_3d(nx=128, ny=96, nz=96, D=10.0, center=(48.0, 47.6, 48.3), storage=cf.STORE_F32)
 results(case, 1, 9, False)
 """, ILBM_OVERLAP_BYTES="0")
+
+
+def test_a_setting_that_is_not_used_takes_no_memory():
+    # IVC forces once whatever loop_ns says; three doubles per marker and
+    # iteration would be 10^12 bytes here
+    import numpy as np
+    from ilbmrex_amd import config as cf
+    from ilbmrex_amd.native import Level
+    case = cf.cylinder_2d(nx=96, ny=64, D=16.0, xc=32.0, yc=32.0, coupling=cf.COUPLING_IVC)
+    out = []
+    for loops in (1, 2 ** 31 - 1):
+        with Level(case.replace(loop_ns=loops), cf.uniform_init(case, u=(case.U0, 0.0, 0.0))) as lev:
+            lev.advance(5, want_state=True)
+            out.append((lev.f(), lev.force_history()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
