@@ -1035,7 +1035,7 @@ int ilbm_box_sums_workspace(const int vlo[3], const int vhi[3], int ncomp, int64
   int64_t cells = 1;
   for (int e = 0; e < 3; ++e) {
     if (vhi[e] < vlo[e]) return ILBM_ERR_INVALID;
-    cells *= vhi[e] - vlo[e] + 1;
+    cells *= (int64_t)vhi[e] - vlo[e] + 1;
   }
   *bytes = 8 * ncomp * ((cells + 255) / 256 + 1);
   return ILBM_OK;
@@ -1044,7 +1044,7 @@ int ilbm_box_sums_workspace(const int vlo[3], const int vhi[3], int ncomp, int64
 int ilbm_box_sums(const ilbm_fab* fab, int comp, int ncomp, const int vlo[3], const int vhi[3], void* work,
                   int64_t work_bytes, double* host_out, void* stream) {
   int64_t need = 0;
-  if (!fab || !fab->p || !work || !host_out || comp < 0 || ncomp < 1 || ncomp > 64 || comp + ncomp > fab->ncomp ||
+  if (!fab || !fab->p || !work || !host_out || comp < 0 || ncomp < 1 || ncomp > 64 || comp > fab->ncomp - ncomp ||
       ilbm_box_sums_workspace(vlo, vhi, ncomp, &need) != ILBM_OK || work_bytes < need)
     return ILBM_ERR_INVALID;
   return guarded([&] {
