@@ -422,8 +422,14 @@ __global__ void __launch_bounds__(256) k_box_fill_patch(Fab S, Fab D, BoxGeom G,
     for (int n = 0; n < nc; ++n) D.p[o + n * D.ns] = 0.0;
     return;
   }
-  if (P.kind == 0 || (meso && P.kind == BC_USER_1)) {
+  if (P.kind == 0) {
     copy_comps(S, p, D, o, nc);
+    return;
+  }
+  // the mesoscopic functors set the populations: components after them stay zero
+  if (meso && P.kind == BC_USER_1) {
+    copy_comps(S, p, D, o, LAT::Q);
+    for (int n = LAT::Q; n < nc; ++n) D.p[o + n * D.ns] = 0.0;
     return;
   }
   if (!meso) {  // macroBcFill
@@ -443,7 +449,7 @@ __global__ void __launch_bounds__(256) k_box_fill_patch(Fab S, Fab D, BoxGeom G,
   meso_ghost<LAT>(P.kind, P.b, fnp, out);
 #pragma unroll
   for (int q = 0; q < LAT::Q; ++q) D.p[o + q * D.ns] = out[q];
-  for (int n = LAT::Q; n < nc; ++n) D.p[o + n * D.ns] = P.sv ? S.p[p + n * S.ns] : 0.0;
+  for (int n = LAT::Q; n < nc; ++n) D.p[o + n * D.ns] = 0.0;
 }
 
 template <class LAT>

@@ -322,7 +322,8 @@ int ilbm_box_fill_patch(const ilbm_case_desc* desc, const ilbm_fab* src, ilbm_fa
                         const int valid_lo[3], const int valid_hi[3], void* stream);
 /* ilbm_box_fill_patch (mesoscopic) of src into dst, ilbm_box_collide of dst
  * and ilbm_box_fill_periodic of dst in one pass; with ghosts == 0 only dst's
- * valid cells are written. */
+ * valid cells are written.  Only the q populations of src and dst are read
+ * and written. */
 int ilbm_box_fill_collide(const ilbm_case_desc* desc, const ilbm_fab* src, ilbm_fab* dst, const ilbm_fab* macro,
                           const ilbm_fab* force, int ghosts, const int valid_lo[3], const int valid_hi[3],
                           void* stream);
