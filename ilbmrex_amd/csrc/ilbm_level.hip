@@ -609,6 +609,7 @@ struct Level {
   double* mout = nullptr;
   double* fout = nullptr;
   bool state_valid = false;
+  int step_path = 0;            // ilbm_level_step_path
   HostCopy host_copy;
   // histories
   double* mass_dev = nullptr;
@@ -2272,6 +2273,7 @@ struct Level {
     }
     state_valid = false;
     const bool body = body_ok && !timing;
+    step_path = body ? 4 : !split ? 1 : ring_ok ? 3 : 2;
     if (body) advance_body(nsteps, want_state);
     for (int s = 0; s < nsteps && !body; ++s) {
       const double time = t_new;  // timeStepWithSubcycling, AmrCoreLBM.cpp:1730-1733
@@ -2635,6 +2637,12 @@ int ilbm_level_set_timing(ilbm_level* h, int enable) {
 int ilbm_level_set_overlap(ilbm_level* h, int enable) {
   if (!h) return ILBM_ERR_INVALID;
   h->L.overlap = enable != 0;
+  return ILBM_OK;
+}
+
+int ilbm_level_step_path(ilbm_level* h, int* path) {
+  if (!h || !path) return ILBM_ERR_INVALID;
+  *path = h->L.step_path;
   return ILBM_OK;
 }
 

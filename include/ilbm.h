@@ -153,6 +153,11 @@ int ilbm_level_set_timing(ilbm_level* L, int enable);
  * way; Sum(Rho) is summed in another order.  No counterpart in the
  * reference. */
 int ilbm_level_set_overlap(ilbm_level* L, int enable);
+/* How the last ilbm_level_advance stepped: 0 none yet, 1 on one stream, 2 and
+ * 3 overlapped in two and three regions, 4 with body tiles (a fixed 2D body's
+ * forcing inside the stream-collide launch).  No counterpart in the
+ * reference. */
+int ilbm_level_step_path(ilbm_level* L, int* path);
 
 /* Measurement helper (no counterpart in the reference): average time of a
  * plain device copy of `bytes` bytes over `iters` launches, used to state
