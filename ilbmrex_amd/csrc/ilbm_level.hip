@@ -524,6 +524,31 @@ constexpr int kBodyLds = 20 * 1024;
 // 18.0, 1000x1000 22 / 31, 2000x1000 37 / 44, 2400x1250 54 / 52, 2000x2000
 // 69 / 67; FP16-shifted 2000x1000 32 / 43, 2400x2000 72 / 56.
 constexpr int64_t kBodyReducedCells = (int64_t)5 << 19;
+// The record of a step with body tiles is one block that walks the whole
+// band, so a wide body's step takes as long as that block, where the
+// separate kernels sum the band in many.  Both sides in us per step, fitted
+// to 829 pairs of measurements (bodies 32 to 275 cells wide, levels of 0.005
+// to 2.4 M cells, every coupling, one to three iterations, three storages;
+// the choice is within 6 % of the faster side):
+//   tiles:    7 + 0.245 per 256 band cells + 1.8 per further iteration, + 8
+//             for an IVC body's second launch;
+//   separate: 20 (FP64) or 18, + 11 per further iteration, + 7.5 for IVC,
+//             + 2.5 for the diagonal, + 4 (FP64) or 10 where the ghost slabs
+//             are a launch of their own, + 21 (FP64), 10.5 (FP32) or 7.5 per
+//             million cells of the level.
+// FP64 500x400, one iteration, tiles / separate: D = 90 16.7 / 24.5, 120 22.4
+// / 25.1, 150 30.0 / 24.2, 200 47.4 / 24.0, 275 81.6 / 26.0; 1000x1000, D =
+// 150 36.6 / 45.4, 200 53.1 / 45.1; FP32 500x400, D = 90 15.7 / 19.6, 120
+// 21.4 / 19.5, 275 80.8 / 21.6.
+static bool body_tiles_pay(int64_t band_cells, int64_t cells, int storage, int loops, bool ivc, bool diag,
+                           bool own_slabs) {
+  const bool f64 = storage == 0;
+  const double tiles = 7.0 + 0.245 * (double)((band_cells + 255) / 256) + 1.8 * (loops - 1) + (ivc ? 8.0 : 0.0);
+  const double separate = (f64 ? 20.0 : 18.0) + 11.0 * (loops - 1) + (ivc ? 7.5 : 0.0) + (diag ? 2.5 : 0.0) +
+                          (own_slabs ? (f64 ? 4.0 : 10.0) : 0.0) +
+                          1e-6 * (double)cells * (f64 ? 21.0 : storage == 1 ? 10.5 : 7.5);
+  return tiles <= separate;
+}
 
 struct Level {
   ilbm_case_desc c{};
@@ -1070,10 +1095,11 @@ struct Level {
   }
 
   // Tables of the body tiles of a fixed 2D body (ILBM_BODY_TILES=0 keeps the
-  // separate forcing kernels).  A body they cannot hold -- stencils beyond
-  // the ghost layers, lists over the LDS budget, more iterations than
-  // kBodyLoops -- and large levels of reduced storage keep the separate
-  // kernels too, and so does a level without memory left for the tables:
+  // separate forcing kernels, =1 takes tiles where body_tiles_pay would not).
+  // A body they cannot hold -- stencils beyond the ghost layers, lists over
+  // the LDS budget, more iterations than kBodyLoops -- large levels of
+  // reduced storage and bodies too wide for the record's one block
+  // (body_tiles_pay) keep the separate kernels too, and so does a level without memory left for the tables:
   // advance never starts on part of them.
   void setup_body() {
     body_tried = true;
@@ -1095,6 +1121,9 @@ struct Level {
     if (c.dim != 2 || moving || cf || !stepbodyfn || n_ne == 0 || nloop > kBodyLoops || (e && e[0] == '0')) return;
     if (c.n[0] > 0xffff || c.n[1] > 0x7fff) return;   // packed cells
     if (st != 0 && ncells > kBodyReducedCells) return;
+    if (!(e && e[0] == '1') && !body_tiles_pay(band_cells, ncells, st, nloop, c.coupling_method == 1, c.coupling_method == 2,
+                                               !wrap && !gfuse))
+      return;
     std::vector<int> where(band_cells, -1);   // list index of a band cell
     for (int ci = 0; ci < n_ne; ++ci) where[ne_h[ci]] = ci;
     auto list_cell = [&](const int p[2]) {
