@@ -1124,32 +1124,41 @@ struct Level {
     if (!(e && e[0] == '1') && !body_tiles_pay(band_cells, ncells, st, nloop, c.coupling_method == 1, c.coupling_method == 2,
                                                !wrap && !gfuse))
       return;
+    const int rec_lds = (int)(64 * ((band_cells + 255) / 256));   // the record's wave sums
+    if (rec_lds > kBodyLds) return;
     std::vector<int> where(band_cells, -1);   // list index of a band cell
     for (int ci = 0; ci < n_ne; ++ci) where[ne_h[ci]] = ci;
     auto list_cell = [&](const int p[2]) {
       const int bi = p[0] - band_lo[0], bj = p[1] - band_lo[1];
       return (bi < 0 || bi >= band_n[0] || bj < 0 || bj >= band_n[1]) ? -1 : where[(size_t)bj * band_n[0] + bi];
     };
-    // stencil points of every marker: list index, or the ghost cell
+    // stencil points of a marker: list index, or the ghost cell; worked out
+    // when a tile first needs them (false: not for tiles)
     struct Pt { int li; int p[2]; };
-    std::vector<Pt> st(25 * (size_t)nm);
-    for (int m = 0; m < nm; ++m)
+    std::vector<Pt> st;
+    std::vector<int> st0(nm, -1);   // a marker's first point
+    auto stencil = [&](int m) {
+      if (st0[m] >= 0) return true;
+      st0[m] = (int)st.size();
+      st.resize(st.size() + 25);
       for (int t = 0; t < 25; ++t) {
-        Pt& q = st[(size_t)m * 25 + t];
+        Pt& q = st[st0[m] + t];
         bool ghost = false;
         int w[2];
         for (int d = 0; d < 2; ++d) {
           const int b = (int)std::floor((xm_h[(size_t)d * nm + m] - c.plo[d]) / c.dx[d]) - ioff[d];
           const int p = b + (d == 0 ? t / 5 : t % 5) - 2;
-          if (p < -2 || p > c.n[d] + 1) return;
+          if (p < -2 || p > c.n[d] + 1) return false;
           q.p[d] = w[d] = p;
           if (p >= 0 && p <= c.n[d] - 1) continue;
           if (c.periodic[d]) w[d] += (p < 0) ? c.n[d] : -c.n[d];
           else ghost = true;
         }
         q.li = ghost ? -1 : list_cell(w);
-        if (!ghost && q.li < 0) return;
+        if (!ghost && q.li < 0) return false;
       }
+      return true;
+    };
     std::map<std::pair<int, int>, std::vector<int>> own;   // list cells of each tile
     for (int ci = 0; ci < n_ne; ++ci)
       own[{ne_h[ci] / band_n[0] / kBodyTile, ne_h[ci] % band_n[0] / kBodyTile}].push_back(ci);
@@ -1162,8 +1171,6 @@ struct Level {
     for (const auto& to : own) {
       BodyTile T{};
       std::vector<int> lc = to.second, lm;
-      std::fill(cslot.begin(), cslot.end(), -1);
-      std::fill(mslot.begin(), mslot.end(), -1);
       for (size_t x = 0; x < lc.size(); ++x) cslot[lc[x]] = (int)x;
       T.nown = (int)lc.size();
       for (int it = nloop - 1; it >= 0; --it) {
@@ -1171,15 +1178,20 @@ struct Level {
         const size_t c1 = lc.size(), m1 = lm.size();
         for (size_t x = 0; x < c1; ++x)
           for (int en = nee_h[lc[x]]; en < nee_h[n_ne + lc[x]]; ++en)
-            if (mslot[em_h[en]] < 0) { mslot[em_h[en]] = (int)lm.size(); lm.push_back(em_h[en]); }
+            if (mslot[em_h[en]] < 0) {
+              if (!stencil(em_h[en])) return;
+              mslot[em_h[en]] = (int)lm.size();
+              lm.push_back(em_h[en]);
+            }
         for (size_t y = m1; y < lm.size(); ++y)
           for (int t = 0; t < 25; ++t) {
-            const int li = st[(size_t)lm[y] * 25 + t].li;
+            const int li = st[st0[lm[y]] + t].li;
             if (li >= 0 && cslot[li] < 0) { cslot[li] = (int)lc.size(); lc.push_back(li); }
           }
         T.nmk[it] = (int)lm.size();
         T.ncell[it] = (int)lc.size();
       }
+      if (body_tile_lds(T) > kBodyLds) return;   // (the lists below only add to it)
       const int nc = (int)lc.size(), nmk = (int)lm.size();
       T.cell0 = (int)rest.size(); T.mk0 = (int)mk.size(); T.pt0 = (int)pt.size();
       T.gh0 = (int)gh.size(); T.ep0 = (int)ep.size(); T.ent0 = (int)em.size();
@@ -1200,7 +1212,7 @@ struct Level {
       std::map<std::pair<int, int>, int> gslot;
       for (int t = 0; t < 25; ++t)
         for (int y = 0; y < nmk; ++y) {
-          const Pt& q = st[(size_t)lm[y] * 25 + t];
+          const Pt& q = st[st0[lm[y]] + t];
           if (q.li >= 0) { pt.push_back(cslot[q.li]); continue; }
           auto ins = gslot.emplace(std::make_pair(q.p[0], q.p[1]), nc + T.ngh);
           if (ins.second) {
@@ -1225,12 +1237,15 @@ struct Level {
       ep.push_back(T.nent);
       if (nc + T.ngh > 0xffff || nmk > 0xffff) return;
       lds = std::max(lds, body_tile_lds(T));
+      if (lds > kBodyLds) return;
       tiles.push_back(T);
+      for (int li : lc) cslot[li] = -1;
+      for (int m : lm) mslot[m] = -1;
     }
+    if (std::find(owned.begin(), owned.end(), 0) != owned.end()) return;   // a marker that no tile evaluates
     for (BodyTile& T : tiles) T.cell0 += (int)cells.size();
     cells.insert(cells.end(), rest.begin(), rest.end());
-    lds = std::max(lds, (int)(64 * ((band_cells + 255) / 256)));   // the record's wave sums
-    if (lds > kBodyLds) return;
+    lds = std::max(lds, rec_lds);
     std::vector<unsigned char> mask(band_cells, 0);
     for (int b : ne_h) mask[b] = 1;
     std::vector<int> ints;

@@ -36,3 +36,24 @@ def test_path_and_results(monkeypatch, n, D, f64, reduced, storage):
     other, ref = _run(c)
     assert {path, other} == {"body tiles", "one stream"}
     assert all(np.array_equal(a, b) for a, b in zip(got, ref))
+
+
+def test_a_refused_body_does_not_pay_for_the_tables(monkeypatch):
+    """Markers too dense for a tile's lists are refused at the first tile: the
+    first advance takes no longer than without tiles by a millisecond (the
+    tables of all 20,000 markers take four)."""
+    import time
+
+    from ilbmrex_amd.native import Level
+    c = cf.cylinder_2d(nx=300, ny=150, D=60.0, xc=100.0, yc=75.0).replace(n_marker=20000)
+    init = cf.uniform_init(c, u=(c.U0, 0.0, 0.0))
+    best = {}
+    for tiles in ("0", "1") * 4:
+        monkeypatch.setenv("ILBM_BODY_TILES", tiles)
+        with Level(c, init) as lev:
+            t = time.perf_counter()
+            lev.advance(1)
+            best[tiles] = min(best.get(tiles, 1.0), time.perf_counter() - t)
+            assert lev.step_path() == "one stream"
+    print(f"[body] first advance {best}", flush=True)
+    assert best["1"] - best["0"] < 1e-3
