@@ -929,18 +929,49 @@ struct Level {
   // 1 decides otherwise): 3D levels whose stored rows are an odd number of
   // 32-cell pieces, so that the row tiling (a wavefront per 64 cells of a
   // row) idles at least half a wavefront per row -- in FP16-shifted storage,
-  // whose kernel is bound by instruction issue, at any size; in FP32 and FP64
-  // on rows of one piece and on large levels.  k_step in us, rows -> linear:
-  // FP16-shifted 160^3 77 -> 62, 200x160x160 sphere 100 -> 88, 96^3 18.4 ->
-  // 15.8 (rows of whole wavefronts lose: duct 48x112x112 19.1 -> 22.1); duct
-  // 24x96x96 FP64 41.6 -> 29.7, FP16-shifted 14.1 -> 11.4; FP32 160^3 112.5
-  // -> 107.4, 130x160x160 117 -> 110, 145x120x120 65.6 -> 65.8, 90x96x96 29.6
-  // -> 31.1; FP64 200^3 440 -> 423, 150x120x120 126.4 -> 126.7.
+  // whose kernel is bound by instruction issue, on rows of any length; in
+  // FP32 and FP64 on rows of one piece and on large levels.  k_step in us,
+  // rows -> linear (D3Q19): FP16-shifted 160^3 77 -> 62, 200x160x160 sphere
+  // 100 -> 88, 96^3 18.4 -> 15.8, 288x64x64 32 -> 21 (rows of whole
+  // wavefronts lose: duct 48x112x112 19.1 -> 22.1); duct 24x96x96 FP64 41.6
+  // -> 29.7, FP16-shifted 14.1 -> 11.4; FP32 160^3 112.5 -> 107.4,
+  // 130x160x160 117 -> 110, 145x120x120 65.6 -> 65.8, 90x96x96 29.6 -> 31.1;
+  // FP64 200^3 440 -> 423, 150x120x120 126.4 -> 126.7.  D3Q27 follows it.
+  //
+  // The row tiling stays (ratios linear / rows of a step, over D3Q19 and
+  // D3Q27 with no walls, in x, in y and z and in all three):
+  // * up to 1024 row blocks of one row each, a row for every SIMD of the chip:
+  //   the linear launch leaves CUs empty there.  32 rows squared 1.01-1.17 in
+  //   every storage, 36 squared FP64 24x36x36 0.82-0.99, FP16-shifted
+  //   160x36x36 0.94-1.04; rows past 256 cells take two blocks each:
+  //   352x20x20 0.91-1.14, 352x28x28 0.84-0.92.  (FP64 rows of 8 cells, one
+  //   64-byte part, gain at any size: 8x32x32 0.79-0.97.)  FP32 and
+  //   FP16-shifted rows of one piece turn at twice that: 24x44x44 0.98-1.06,
+  //   24x48x48 0.93-1.02, 24x64x64 0.85-0.99;
+  // * on all-periodic FP32 and FP64 levels of more than 256 K stored cells
+  //   whose one-piece rows end inside a 64-byte part of a line (28x160x160
+  //   1.16-1.20, FP32 24x96x96 1.08; 16x160x160 0.68-0.97);
+  // * in D3Q19 FP16-shifted storage with walls in y or z, on rows whose
+  //   blocks the row tiling fills with 256 threads (96 and 224 cells stored:
+  //   66x96x96 1.06, 200x128x128 with all walls 1.07; 160 stored, blocks of
+  //   192: 0.95-1.02), and with walls in x too on longer rows of which at
+  //   most an eighth is idle (480x110x110 1.08; 416x96x96 0.93).
   bool linear_steps() const {
-    if (c.dim != 3 || g.js * c.n[1] * c.n[2] >= ((int64_t)1 << 31) - kBlock) return false;
+    const int64_t stored = g.js * c.n[1] * c.n[2];
+    if (c.dim != 3 || stored >= ((int64_t)1 << 31) - kBlock) return false;
     if (const char* e = std::getenv("ILBM_STEP_LINEAR")) return e[0] == '1';
     if (g.js % 64 == 0) return false;
-    return st == 2 || g.js <= 32 || ncells >= kLinCells;
+    const bool one_piece = g.js <= 32;
+    if (!one_piece && st != 2) return ncells >= kLinCells;
+    const int64_t row_blocks = (int64_t)c.n[1] * c.n[2] * grid.x;
+    if (row_blocks <= (one_piece && st != 0 ? 2048 : 1024) && !(st == 0 && c.n[0] == 8)) return false;
+    if (st != 2) {
+      const bool periodic = !(nonper[0] || nonper[1] || nonper[2]);
+      return !(periodic && stored > 256 * 1024 && c.n[0] * popbytes % 64 != 0);
+    }
+    if (lat != 1 || one_piece || !(nonper[1] || nonper[2]) || block.x * block.y != (unsigned)kBlock) return true;
+    const int64_t lanes = (int64_t)block.x * grid.x;
+    return c.n[0] > 256 && !(nonper[0] && 8 * (lanes - g.js) <= lanes);
   }
 
   // number of blocks of a tile of width bx (height kBlock / bx)
