@@ -500,14 +500,6 @@ static int64_t plane_stride(int64_t cells, int64_t pop_bytes) {
 constexpr int kFarBlocksPerCu = 0;
 constexpr int kFarAfter = 0;
 constexpr int kRingStream = 0;   // Level::RING_NEAR
-// Population bytes of a step from which an IB level overlaps its far cells.
-// Sphere steps in us, overlapped / on one stream: 161x101x99 FP64 (489 MB)
-// 133 / 146, FP32 (245 MB) 78 / 72, FP16-shifted 62 / 53; 192x112x112 FP64
-// 167 / 183, FP32 (366 MB) 89 / 90, FP16-shifted (183 MB) 58 / 59;
-// 256x128x128 FP32 (637 MB) 122 / 125, FP16-shifted (319 MB) 77 / 75.
-// ILBM_OVERLAP_BYTES overrides it.
-constexpr int64_t kOverlapBytes = (int64_t)350 << 20;
-
 // FP32 and FP64 levels from this many cells may step in linear blocks
 // (Level::linear_steps).
 constexpr int64_t kLinCells = (int64_t)3 << 20;
@@ -1939,6 +1931,56 @@ struct Level {
     }
   }
 
+  // Population bytes of a step (read and written) from which an IB level
+  // overlaps its far cells; ILBM_OVERLAP_BYTES overrides it.  Below, the
+  // host's time to queue an overlapped step (60-75 us) and the cross-stream
+  // waits cost more than the overlap saves.  Measured on 900 spheres and
+  // cylinders, 1 to 12 M cells; us per step, overlapped / on one stream, of
+  // bodies 20 cells wide:
+  // * 3D: D3Q19 FP32 128x144x144 (403 MB) 86 / 86, 256x104x104 (421 MB) 89 /
+  //   90, 224x88x88 (264 MB) 68 / 64; FP64 128x96x96 (359 MB) 107 / 102,
+  //   128x120x120 (560 MB) 116 / 130; FP16-shifted 256x120x120 (280 MB) 67 /
+  //   67, 160x144x144 (252 MB) 72 / 67; D3Q27 FP32 224x104x104 (523 MB) 109 /
+  //   110, FP16-shifted 256x104x104 (299 MB) 75 / 74;
+  // * 3D, rows of 129 to 192 cells in the row tiling, whose blocks do not hold
+  //   the record's 256 threads: on one stream the record is a launch of its
+  //   own in the chain.  FP32 D3Q19 192x104x104 (316 MB) 88 / 80, 150x120x120
+  //   (328 MB) 83 / 87; D3Q27 192x88x88 (321 MB) 92 / 85, 150x104x104 (350 MB)
+  //   92 / 95; FP16-shifted D3Q19 192x104x104 (158 MB) 61 / 54, 192x144x144
+  //   (303 MB) 71 / 78; D3Q27 192x88x88 (161 MB) 61 / 56, 180x104x104 (210 MB)
+  //   63 / 68.  FP16-shifted rows past 256 cells in the row tiling, where a
+  //   second block is partly idle, are alike: D3Q19 320x88x88 (188 MB) 65 /
+  //   67, 384x104x104 (316 MB) 84 / 86;
+  // * 3D FP16-shifted with several iterations, in D3Q27 or linear blocks:
+  //   D3Q19 160x120x120 (175 MB) 96 / 100, D3Q27 160x104x104 (187 MB) 102 /
+  //   106, 160x144x144 (358 MB) 116 / 138; but D3Q19 192x144x144 in rows (303
+  //   MB) 126 / 117, FP32 D3Q27 192x104x104 (449 MB) 155 / 149.  IVC bodies of
+  //   these classes: D3Q27 192x104x104 (224 MB) 71 / 72, D3Q19 160x144x144
+  //   (252 MB) 67 / 74, D3Q27 256x104x104 (299 MB) 76 / 79; others D3Q19
+  //   192x144x144 (303 MB) 88 / 82, FP32 160x120x120 (350 MB) 96 / 90;
+  // * 2D: FP16-shifted 2000x2000 (144 MB) 59 / 54, 3000x2000 (216 MB) 67 / 73,
+  //   4000x2000 (288 MB) 80 / 90; FP32 2400x1250 (216 MB) 63 / 58, 2000x2000
+  //   (288 MB) 69 / 71, with two iterations 74 / 80; FP64 2000x2000 (576 MB)
+  //   123 / 122.
+  // A near box of more than a 64th of the cells (a 32nd in FP16-shifted
+  // storage with one iteration) takes the overlap's gain: 36 cells wide, FP32
+  // 150x120x120 105 / 97, D3Q27 150x104x104 120 / 106, FP16-shifted D3Q27
+  // 192x104x104 83 / 79; 32 wide with two iterations, FP16-shifted D3Q27
+  // 256x104x104 134 / 121 (12 wide: 75 / 83, 86 / 94, 65 / 65, 104 / 116).
+  int64_t overlap_bytes() const {
+    constexpr int64_t MiB = (int64_t)1 << 20;
+    int64_t near = 1;
+    for (int d = 0; d < c.dim; ++d) near *= band_n[d] + 2;
+    if ((st == 2 && async_record() ? 32 : 64) * near > ncells) return 350 * MiB;
+    if (c.dim == 2) return (st == 2 ? 176 : st == 1 ? 256 : 350) * MiB;
+    const bool slab_launch = !wrap && !gfuse;   // the record goes with it
+    const bool own_record = !slab_launch && step_block.x * step_block.y != (unsigned)kSumsBlock;
+    if (!async_record()) return (st == 2 && (lat == 2 || step_lin) ? 160 : 350) * MiB;
+    if (c.coupling_method == 1) return (st == 2 && (lat == 2 || step_lin) ? 220 : 350) * MiB;
+    if (st == 2) return (own_record || (c.n[0] > 256 && !step_lin) ? 176 : 350) * MiB;
+    return (own_record ? 310 : 350) * MiB;
+  }
+
   // the near box (IB band grown by one cell; the whole extent of a periodic
   // dimension it would wrap across) and the resources of the overlapped step
   bool split_ready() {
@@ -1946,11 +1988,8 @@ struct Level {
     // below ~1M cells the two cross-stream waits per step cost more than
     // the overlap saves (512x256 D2Q9 FP64: 2.5 -> 1.9 GLUPS with it)
     if (ncells < ((int64_t)1 << 20)) return false;
-    // and so they do where the far cells' launch is shorter than the host
-    // needs to queue an overlapped step (60-75 us): under kOverlapBytes of
-    // populations read and written per step
     const char* ob = std::getenv("ILBM_OVERLAP_BYTES");
-    if (ncells * 2 * c.q * (int64_t)popbytes < (ob ? (int64_t)std::atoll(ob) : kOverlapBytes)) return false;
+    if (ncells * 2 * c.q * (int64_t)popbytes < (ob ? (int64_t)std::atoll(ob) : overlap_bytes())) return false;
     if (!stream_b) {
       int per_cu = kFarBlocksPerCu;
       if (const char* e = std::getenv("ILBM_FAR_BLOCKS_PER_CU")) per_cu = std::max(0, std::atoi(e));
