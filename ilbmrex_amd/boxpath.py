@@ -177,32 +177,33 @@ class BoxLevel:
                 a.free()
 
     # -- FillPatch ---------------------------------------------------------
+    def _fill_macros(self, time, coarse: Optional["BoxLevel"]):
+        """smSborder at `time`; lev > 0: own valid cells, and the ghost cells of
+        smSborder and sfSborder from the coarse level."""
+        L, d, lo, hi = self.L, self._d, self._lo, self._hi
+        if coarse is None:
+            self._check(L.ilbm_box_fill_patch(d, self.m_old.ref(), self.smS.ref(), 0, lo, hi, None), "box_fill_patch")
+            return
+        self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
+                                             time, self.sfS.ref(), self.smS.ref(), self.m_old.ref(), self.nmac,
+                                             lo, hi, None), "box_cf_fill_patch")
+
     def fill_patch(self, time, coarse: Optional["BoxLevel"] = None):
         """sfSborder / smSborder of a step starting at `time`, before the
         collision (advance_level collides in the same pass)."""
         L, d, lo, hi = self.L, self._d, self._lo, self._hi
         if coarse is None:
             self._check(L.ilbm_box_fill_patch(d, self.f_old.ref(), self.sfS.ref(), 1, lo, hi, None), "box_fill_patch")
-            self._check(L.ilbm_box_fill_patch(d, self.m_old.ref(), self.smS.ref(), 0, lo, hi, None), "box_fill_patch")
-            return
-        self._check(L.ilbm_box_copy(self.f_old.ref(), self.sfS.ref(), lo, hi, self.q, None), "box_copy")
-        self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
-                                             time, self.sfS.ref(), self.smS.ref(), self.m_old.ref(), self.nmac,
-                                             lo, hi, None), "box_cf_fill_patch")
+        else:
+            self._check(L.ilbm_box_copy(self.f_old.ref(), self.sfS.ref(), lo, hi, self.q, None), "box_copy")
+        self._fill_macros(time, coarse)
 
     # -- one AdvancePhiAtLevel ------------------------------------------------
     def advance_level(self, time, coarse: Optional["BoxLevel"] = None):
         self.f_new, self.f_old = self.f_old, self.f_new
         self.m_new, self.m_old = self.m_old, self.m_new
         L, d, lo, hi = self.L, self._d, self._lo, self._hi
-        if coarse is None:
-            self._check(L.ilbm_box_fill_patch(d, self.m_old.ref(), self.smS.ref(), 0, lo, hi, None), "box_fill_patch")
-        else:
-            # FillPatchMacro / FillPatchMesoscopic for lev > 0: own valid
-            # cells, ghosts from the coarse level at `time`
-            self._check(L.ilbm_box_cf_fill_patch(d, coarse.m_old.ref(), coarse.m_new.ref(), coarse.t_old, coarse.t_new,
-                                                 time, self.sfS.ref(), self.smS.ref(), self.m_old.ref(), self.nmac,
-                                                 lo, hi, None), "box_cf_fill_patch")
+        self._fill_macros(time, coarse)
         force = None
         if self.has_force:
             u = self.uniform_force

@@ -1596,7 +1596,7 @@ __global__ void __launch_bounds__(kBlock) k_step_record(StepArgs a, uint32_t tx,
 // k_ib_interp, k_ib_ivc_*, k_ib_spread_t, k_ib_correct, k_ib_export_fixup and
 // k_sums_record term by term and in their order: the results are the same
 // bits.  An IVC body needs all markers between interpolation and spreading:
-// its tiles stop at the right-hand side and k_body_ivc does the rest.
+// its tiles stop at the right-hand side and k_body's MODE 2 does the rest.
 // ---------------------------------------------------------------------------
 constexpr int kBodyTile = 8;
 constexpr int kBodyOwn = kBodyTile * kBodyTile;   // a tile's own cells, at most (whole wavefronts)

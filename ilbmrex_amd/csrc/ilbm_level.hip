@@ -322,7 +322,7 @@ static void launch_step(dim3 g, dim3 b, hipStream_t s, const StepArgs& a, hipEve
   check_step_block(b);
   const uint32_t nt = g.x * g.y * g.z;
   if constexpr (LAT::D == 3) {
-    if (a.lin && a.sub_mode < 2) {   // 256 x 1 blocks
+    if (a.lin && a.sub_mode < 2) {   // 256 x 1 blocks, never the persistent launch
       if (e0) hipExtLaunchKernelGGL((k_step<LAT, ST, AM, true>), g, b, 0, s, e0, e1, 0, a);
       else hipLaunchKernelGGL((k_step<LAT, ST, AM, true>), g, b, 0, s, a);
       return;
