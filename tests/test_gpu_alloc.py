@@ -19,7 +19,9 @@ static int left = 0;
 extern "C" void refuse(int k) { left = k; }           // the k-th allocation from now
 extern "C" int pending() { return left; }
 extern "C" int hipMalloc(void** p, size_t n) {
-  static auto real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), "hipMalloc");
+  static void* hip = dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD);   // as the framework loaded it
+  if (!hip) return 2;
+  static auto real = (int (*)(void**, size_t))dlsym(hip, "hipMalloc");
   return real(p, left > 0 && --left == 0 ? (size_t)1 << 60 : n);   // more than there is
 }
 """
